@@ -28,13 +28,8 @@
 #include "mfma_common.hpp"
 #include "q8k_block.hpp"
 
-#include <algorithm>
 #include <atomic>
 #include <cstdlib>
-#include <functional>
-#include <queue>
-#include <utility>
-#include <vector>
 
 namespace barq {
 
@@ -511,415 +506,9 @@ void attn_combine_q8k_kernel(const float* __restrict__ part, int n_split, int n_
     }
 }
 
-// Position blocks of 32 that query block qb sees (am_qblock's range).
-__host__ __device__ __forceinline__ int am_qblock_blocks(int qb, int q_len, int kv_len, long long start_pos) {
-    const int i_last = qb * 32 + 31 < q_len - 1 ? qb * 32 + 31 : q_len - 1;
-    const long long vis_last = start_pos + i_last + 1;
-    const int j_end = (int)(vis_last < kv_len ? vis_last : kv_len);
-    return (j_end + 31) / 32;
-}
-
-// The merge for a few splits (the prompt kernel's): one thread per output
-// value, 256 per workgroup (the 256 / HD heads of one Q8_K block of row i);
-// Q8 writes the block's Q8_K bytes (q8_k_block) instead of the f32 values.
-template <int HD, bool Q8>
-__global__ __launch_bounds__(256)
-void attn_combine_few_kernel(const float* __restrict__ part, int stride, int chunk, int n_head, int q_len, int kv_len,
-                             long long start_pos, float* __restrict__ out, uint8_t* __restrict__ out_q8) {
-    __shared__ __align__(16) float vals[256];
-    const int b = blockIdx.x, i = blockIdx.y, t = threadIdx.x;
-    const int h = b * (256 / HD) + t / HD, d = t % HD;
-    // the pieces of row i's query block (attn_mfma_kernel's list)
-    const int n_split = (am_qblock_blocks(i / 32, q_len, kv_len, start_pos) + chunk - 1) / chunk;
-    const float* pp = part + ((size_t)i * n_head + h) * stride * (HD + 2);
-    float M = -INFINITY;
-    for (int sp = 0; sp < n_split; sp++) M = fmaxf(M, pp[(size_t)sp * (HD + 2)]);
-    float L = 0.0f, O = 0.0f;
-    for (int sp = 0; sp < n_split; sp++) {
-        const float ms = pp[(size_t)sp * (HD + 2)];
-        const float w = ms == -INFINITY ? 0.0f : fast_exp2(ms - M);
-        L = __builtin_fmaf(pp[(size_t)sp * (HD + 2) + 1], w, L);
-        O = __builtin_fmaf(pp[(size_t)sp * (HD + 2) + 2 + d], w, O);
-    }
-    const float v = O / L;
-    if constexpr (!Q8) {
-        out[((size_t)i * n_head + h) * HD + d] = v;
-    } else {
-        vals[t] = v;
-        __syncthreads();
-        if (t < 64) {
-            const float4 v4 = reinterpret_cast<const float4*>(vals)[t];
-            const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
-            q8_k_block(vv, t, out_q8 + ((size_t)i * (n_head * HD / 256) + b) * Q8_K_BYTES);
-        }
-    }
-}
-
 bool attention_supported(size_t head_dim) { return head_dim == 64 || head_dim == 128 || head_dim == 256; }
 
-// ---- prompt chunks on MFMA ----------------------------------------------------
-// For q_len >= 32 (BARQ_ATTN_MFMA_MIN_Q) and head_dim 128 a workgroup covers
-// 32 query rows of W query heads that share one kv head (one wave per head)
-// and walks the visible positions in blocks of 32 with
-// v_mfma_f32_32x32x2_f32 (f32 products and sums, as the VALU path):
-//   S^T[kv, q] = K[kv, :] . Q[q, :]   A = K rows (lane c: row c, dims 64 g ..),
-//                                     B = Q^T (lane c: query c, the same dims)
-//   online softmax per query column: a lane holds 16 positions of its query,
-//   the other 16 sit in lane c ^ 32
-//   O^T[d, q] += V[kv, d] P[q, kv]    B = P^T straight from S^T's registers
-//                                     (step s pairs positions 8(s/4) + s%4 and
-//                                     +4, which lanes c and c + 32 hold as
-//                                     register s); A = V^T with output row i of
-//                                     block b standing for dim 4 i + b, so one
-//                                     16-byte read per lane feeds the four blocks.
-// Each block's K and V rows are copied once per workgroup into LDS by
-// buffer->LDS loads one block ahead (two stages), in rows of 528 bytes (one
-// pad piece: conflict-free fragment reads); rows at or past kv_len read as
-// zero.  Exponentials are base 2 on pre-scaled scores, like the split kernel.
-typedef float f32x16a __attribute__((ext_vector_type(16)));
-constexpr int AM_RS = 528, AM_PIECES = 33, AM_BLK = 32 * AM_RS;
-constexpr int AM_INSTR = (32 * AM_PIECES + 63) / 64;   // load instructions per K or V block (17)
-
-// the buffer->LDS loads of one block (K and V) split over the workgroup's W waves
-template <int W>
-__device__ __forceinline__ void am_issue(uint8_t* stage, i32x4v kr, i32x4v vr, uint32_t soff, int wave, int l) {
-    #pragma unroll
-    for (int q = 0; q < (2 * AM_INSTR + W - 1) / W; q++) {
-        const int idx = q * W + wave;
-        if (idx < 2 * AM_INSTR) {
-            const int kvsel = idx >= AM_INSTR, ii = idx - kvsel * AM_INSTR;
-            const int p = ii * 64 + l, row = p / AM_PIECES, piece = p - row * AM_PIECES;
-            if (p < 32 * AM_PIECES) {
-                const uint32_t voff = (uint32_t)row * 512u + 16u * (uint32_t)(piece < 32 ? piece : 0);
-                lds_load16(kvsel ? vr : kr, stage + kvsel * AM_BLK + 1024 * ii, voff, soff);
-            }
-        }
-    }
-}
-
-// One 32-row query block qb of the workgroup's W heads.  With n_split > 1
-// the workgroup takes split `split` of the block's visible positions (a
-// contiguous run of 32-position blocks) and stores its partial state (max in
-// log2 units, sum, unnormalised output) in the split kernel's layout for the
-// merge kernels; an empty run stores (-inf, 0, 0).
-template <int W>
-__device__ __forceinline__ void am_qblock(uint8_t (&lds)[2][2 * AM_BLK], const float* __restrict__ q,
-                                          const float* __restrict__ kc, const float* __restrict__ vc, size_t layer_off,
-                                          size_t head_stride, int n_head, int n_head_kv, int q_len, int kv_len,
-                                          long long start_pos, float score_scale, float* __restrict__ out, int qb,
-                                          int chunk = 0, int split = 0, int stride = 1,
-                                          float* __restrict__ part = nullptr, int grp = -1) {
-    constexpr int HD = 128;
-    const int l = threadIdx.x & 63, c = l & 31, g = l >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int h = (grp < 0 ? (int)blockIdx.y : grp) * W + wave;
-    const int hk = (int)((long long)h * n_head_kv / n_head);   // the same for the W heads
-    const int i0 = qb * 32, qi = i0 + c;
-    const bool q_ok = qi < q_len;
-
-    const float* kh = kc + layer_off + (size_t)hk * head_stride;
-    const float* vh = vc + layer_off + (size_t)hk * head_stride;
-    const i32x4v kr = make_rsrc4(kh, (uint32_t)kv_len * 512u);
-    const i32x4v vr = make_rsrc4(vh, (uint32_t)kv_len * 512u);
-    const int nblk_all = am_qblock_blocks(qb, q_len, kv_len, start_pos);
-    // chunk > 0: this workgroup takes blocks [split, split + 1) * chunk of
-    // the query block's range and writes a partial state
-    const int b_lo = chunk > 0 ? min(split * chunk, nblk_all) : 0;
-    const int nblk = chunk > 0 ? min(b_lo + chunk, nblk_all) : nblk_all;
-    if (b_lo < nblk) am_issue<W>(lds[0], kr, vr, (uint32_t)b_lo * 32u * 512u, wave, l);
-
-    float qv[64];
-    {
-        const float4* qp = reinterpret_cast<const float4*>(q + ((size_t)h * q_len + (q_ok ? qi : 0)) * HD + 64 * g);
-        #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const float4 t = q_ok ? qp[u] : make_float4(0.f, 0.f, 0.f, 0.f);
-            qv[4 * u] = t.x; qv[4 * u + 1] = t.y; qv[4 * u + 2] = t.z; qv[4 * u + 3] = t.w;
-        }
-    }
-    const long long vis_q = start_pos + qi + 1;   // this lane's query sees positions below vis_q
-
-    f32x16a o0 = {}, o1 = {}, o2 = {}, o3 = {};
-    float m = -INFINITY, lsum = 0.0f;
-    for (int b = b_lo; b < nblk; b++) {
-        const int j0 = 32 * b;
-        wait_vmcnt<0>();
-        asm volatile("" ::: "memory");
-        __syncthreads();   // block b is in its stage; every wave is done with the other one
-        if (b + 1 < nblk) am_issue<W>(lds[(b + 1 - b_lo) & 1], kr, vr, (uint32_t)(j0 + 32) * 512u, wave, l);
-        const uint8_t* ks = lds[(b - b_lo) & 1];
-        const uint8_t* vs = ks + AM_BLK;
-        f32x16a sa = {}, sb = {};
-        #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const float4 kk = *reinterpret_cast<const float4*>(ks + c * AM_RS + 256 * g + 16 * u);
-            sa = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.x, qv[4 * u], sa, 0, 0, 0);
-            sb = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.y, qv[4 * u + 1], sb, 0, 0, 0);
-            sa = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.z, qv[4 * u + 2], sa, 0, 0, 0);
-            sb = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.w, qv[4 * u + 3], sb, 0, 0, 0);
-        }
-        float sc[16];
-        float bm = -INFINITY;
-        #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int kv = j0 + 8 * (r >> 2) + 4 * g + (r & 3);
-            const bool vis = kv < kv_len && kv < vis_q;
-            sc[r] = vis ? (sa[r] + sb[r]) * score_scale : -INFINITY;
-            bm = fmaxf(bm, sc[r]);
-        }
-        {   // with the other half-wave (one gfx950 half-wave swap, no LDS round trip)
-            auto hb = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, bm), __builtin_bit_cast(int, bm), false, false);
-            bm = fmaxf(__builtin_bit_cast(float, (int)hb[0]), __builtin_bit_cast(float, (int)hb[1]));
-        }
-        // Position 0 is visible to every query, so without a split mn is
-        // finite from the first block on; a split that starts later can hold
-        // blocks a query sees none of (mn = -inf): exponents then use 0 as
-        // the reference, so they are 0 instead of NaN and the state stays
-        // (-inf, 0, 0).
-        const float mn = fmaxf(m, bm);
-        const float mref = mn == -INFINITY ? 0.0f : mn;
-        const float corr = fast_exp2(m - mref);   // 0 while m is -inf
-        m = mn;
-        float p[16];
-        float rs = 0.0f;
-        #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            p[r] = fast_exp2(sc[r] - mref);   // 0 for masked positions
-            rs += p[r];
-        }
-        rs = swap32_add(rs, rs);   // + the other half-wave's, as v + v[lane ^ 32]
-        lsum = lsum * corr + rs;
-        o0 *= corr; o1 *= corr; o2 *= corr; o3 *= corr;
-        #pragma unroll
-        for (int st = 0; st < 16; st++) {
-            const int kv = 8 * (st >> 2) + 4 * g + (st & 3);
-            const float4 vv = *reinterpret_cast<const float4*>(vs + kv * AM_RS + 16 * c);
-            o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, p[st], o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, p[st], o1, 0, 0, 0);
-            o2 = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, p[st], o2, 0, 0, 0);
-            o3 = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, p[st], o3, 0, 0, 0);
-        }
-    }
-    if (chunk > 0) {
-        if (q_ok) {
-            float* pp = part + (((size_t)qi * n_head + h) * stride + split) * (HD + 2);
-            if (g == 0) {
-                pp[0] = m;
-                pp[1] = lsum;
-            }
-            #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int i = 8 * (r >> 2) + 4 * g + (r & 3);
-                float* d = pp + 2 + 4 * i;   // 8-byte aligned rows: two float2 stores
-                *reinterpret_cast<float2*>(d) = make_float2(o0[r], o1[r]);
-                *reinterpret_cast<float2*>(d + 2) = make_float2(o2[r], o3[r]);
-            }
-        }
-        return;
-    }
-    if (q_ok) {
-        float* op = out + ((size_t)qi * n_head + h) * HD;
-        #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int i = 8 * (r >> 2) + 4 * g + (r & 3);
-            *reinterpret_cast<float4*>(op + 4 * i) = make_float4(o0[r] / lsum, o1[r] / lsum, o2[r] / lsum, o3[r] / lsum);
-        }
-    }
-}
-
-// Causal prompts leave query block qb with qb + 1 position blocks (plus the
-// cached prefix).  PAIR: workgroup x takes the long block nqb - 1 - x and
-// then the short block x, so every workgroup has about the same work (used
-// when the pairs alone fill the CUs).  Otherwise, with chunk > 0, each query
-// block's range is cut into pieces of chunk blocks, and workgroup x takes
-// piece x of the list that runs from the longest query block down (so no
-// workgroup has more than chunk blocks, whatever the query block); with
-// chunk == 0 workgroup x takes query block nqb - 1 - x whole.
-template <int W, bool PAIR>
-__global__ __launch_bounds__(64 * W)
-void attn_mfma_kernel(const float* __restrict__ q, const float* __restrict__ kc, const float* __restrict__ vc,
-                      size_t layer_off, size_t head_stride, int n_head, int n_head_kv, int q_len, int kv_len,
-                      long long start_pos, float score_scale, float* __restrict__ out, float* __restrict__ part,
-                      int chunk, int stride) {
-    __shared__ __align__(16) uint8_t lds[2][2 * AM_BLK];
-    const int nqb = (q_len + 31) / 32, x = blockIdx.x;
-    if (!PAIR && chunk > 0) {
-        // the list is ordered by length across the head groups: workgroup x
-        // takes piece x / G of head group x % G (G = n_head / W groups; the
-        // grid is one-dimensional here)
-        const int groups = n_head / W;
-        const int grp = x % groups;
-        int qb = nqb - 1, rem = x / groups;
-        for (; qb >= 0; qb--) {
-            const int pieces = (am_qblock_blocks(qb, q_len, kv_len, start_pos) + chunk - 1) / chunk;
-            if (rem < pieces) break;
-            rem -= pieces;
-        }
-        if (qb < 0) return;   // past the list (the grid is its length)
-        am_qblock<W>(lds, q, kc, vc, layer_off, head_stride, n_head, n_head_kv, q_len, kv_len, start_pos, score_scale,
-                     out, qb, chunk, rem, stride, part, grp);
-        return;
-    }
-    const int qb_long = nqb - 1 - x;
-    am_qblock<W>(lds, q, kc, vc, layer_off, head_stride, n_head, n_head_kv, q_len, kv_len, start_pos, score_scale, out,
-                 qb_long);
-    if (PAIR && x < qb_long) {
-        __syncthreads();   // every wave is done with the stages
-        am_qblock<W>(lds, q, kc, vc, layer_off, head_stride, n_head, n_head_kv, q_len, kv_len, start_pos, score_scale,
-                     out, x);
-    }
-}
-
-static int attn_mfma_min_q() { return tuning_env(TUNE_ATTN_MFMA_MIN_Q, 32); }
-
-// The prompt path: head_dim 128, q_len at the threshold, and a kv head's
-// rows addressable by the 32-bit buffer offsets of its K/V loads.
-static bool attn_mfma_path(const AttnArgs& a) {
-    return a.head_dim == 128 && a.q_len >= (size_t)attn_mfma_min_q() && a.kv_len < ((size_t)1 << 23);
-}
-
-static int cu_count_attn();
-
-// Launch plan of the prompt kernel: W query heads per workgroup (W divides
-// the GQA group), query-block pairing when the pairs alone fill the CUs, and
-// otherwise pieces of `chunk` position blocks (partial states merged by
-// attn_combine_few_kernel): chunk is the work per CU if the blocks of all
-// query blocks were shared evenly, so no workgroup runs much longer than the
-// average.  The plan assumes the chunk's queries are the last q_len of the
-// kv_len positions (a prompt); at launch only the piece counts follow the
-// actual start position, within `stride` pieces per query block (the
-// workspace bound).
-struct AmPlan {
-    int w;
-    int chunk;    // position blocks per piece; 0: whole query blocks, no partial states
-    int stride;   // partial states per (query row, head)
-    bool pair;
-    unsigned nqb, groups;
-};
-
-static AmPlan attn_mfma_plan_uncached(size_t n_head, size_t n_head_kv, size_t q_len, size_t kv_len);
-
-// The plan of the last (n_head, n_head_kv, q_len, kv_len, device) this
-// thread asked for: the workspace query and the launch ask in turn.
-static AmPlan attn_mfma_plan(size_t n_head, size_t n_head_kv, size_t q_len, size_t kv_len) {
-    struct Entry {
-        size_t key[4];
-        int dev;
-        AmPlan plan;
-        bool valid;
-    };
-    thread_local Entry last = {{0, 0, 0, 0}, -1, AmPlan{}, false};
-    if (tuning_env(TUNE_ATTN_MFMA_SPLIT) > 0) return attn_mfma_plan_uncached(n_head, n_head_kv, q_len, kv_len);
-    int dev = -1;
-    if (hipGetDevice(&dev) != hipSuccess) dev = -1;
-    if (last.valid && last.dev == dev && last.key[0] == n_head && last.key[1] == n_head_kv && last.key[2] == q_len &&
-        last.key[3] == kv_len)
-        return last.plan;
-    const AmPlan p = attn_mfma_plan_uncached(n_head, n_head_kv, q_len, kv_len);
-    last = Entry{{n_head, n_head_kv, q_len, kv_len}, dev, p, true};
-    return p;
-}
-
-static AmPlan attn_mfma_plan_uncached(size_t n_head, size_t n_head_kv, size_t q_len, size_t kv_len) {
-    AmPlan p{};
-    const size_t grp = (n_head_kv && n_head % n_head_kv == 0) ? n_head / n_head_kv : 1;
-    p.w = grp % 4 == 0 ? 4 : grp % 2 == 0 ? 2 : 1;
-    p.nqb = (unsigned)((q_len + 31) / 32);
-    p.groups = (unsigned)(n_head / p.w);
-    const size_t cus = (size_t)cu_count_attn();
-    p.pair = (size_t)(p.nqb / 2) * p.groups >= cus;
-    p.chunk = 0;
-    p.stride = 1;
-    // the merge writes whole Q8_K blocks (256 values: two heads of 128)
-    if (p.pair || (n_head * 128) % 256 != 0) return p;
-    const long long start = kv_len > q_len ? (long long)(kv_len - q_len) : 0;
-    size_t total = 0;
-    int longest = 0;
-    for (unsigned qb = 0; qb < p.nqb; qb++) {
-        const int nb = am_qblock_blocks((int)qb, (int)q_len, (int)kv_len, start);
-        total += (size_t)nb;
-        longest = nb > longest ? nb : longest;
-    }
-    (void)total;
-    // Choose the chunk by simulating the launch in units of one position
-    // block: the pieces in the kernel's order (each costing its blocks + 1.5
-    // for its fixed part: the query rows, the first copy, the partial state),
-    // every CU holding up to two workgroups that share it equally, each
-    // further piece going to the CU that frees a slot first.  Candidates cut
-    // the longest query block into k = 1 .. 64 pieces; ties keep fewer
-    // pieces.  The model picks the measured best at 512, 768 and 1024 tokens
-    // (Llama-3-8B heads, us per call, chunk: time): 512 tokens 6: 55.5, 3:
-    // 59.3, 8: 61.8, 4: 63.3; 768 tokens 6: 86.2, 12: 97, 4: 97.6, 5: 99.3,
-    // 8: 100, 16: 102.3, 24: 122; 1024 tokens 11: 132, 6: 138, 32 (whole
-    // query blocks): 157.4, 8: 157.6.  (With a fixed part of 1 block it chose
-    // 5 at 768 tokens.)
-    std::vector<int> nbs(p.nqb);
-    for (unsigned qb = 0; qb < p.nqb; qb++) nbs[qb] = am_qblock_blocks((int)qb, (int)q_len, (int)kv_len, start);
-    auto simulate = [&](int c) {
-        std::vector<double> jobs;   // the kernel's order: query blocks longest first, then the head groups
-        for (int qb = (int)p.nqb - 1; qb >= 0; qb--)
-            for (int b = 0; b < nbs[qb]; b += c) {
-                const double len = (nbs[qb] - b < c ? nbs[qb] - b : c) + 1.5;
-                for (unsigned g = 0; g < p.groups; g++) jobs.push_back(len);
-            }
-        struct Cu { double t, w[2]; int n; };
-        std::vector<Cu> cu(cus, Cu{0.0, {0.0, 0.0}, 0});
-        size_t next = 0;
-        for (int pass = 0; pass < 2; pass++)
-            for (size_t k = 0; k < cus && next < jobs.size(); k++) cu[k].w[cu[k].n++] = jobs[next++];
-        auto event = [](const Cu& u) {
-            return u.n == 2 ? u.t + 2.0 * (u.w[0] < u.w[1] ? u.w[0] : u.w[1]) : u.t + u.w[0];
-        };
-        typedef std::pair<double, size_t> Ev;
-        std::priority_queue<Ev, std::vector<Ev>, std::greater<Ev>> heap;
-        for (size_t k = 0; k < cus; k++)
-            if (cu[k].n) heap.push(Ev(event(cu[k]), k));
-        double end = 0.0;
-        while (!heap.empty()) {
-            const Ev ev = heap.top();
-            heap.pop();
-            Cu& u = cu[ev.second];
-            if (u.n == 2) {   // the shorter job ends; the other has done as much
-                const int done = u.w[0] < u.w[1] ? 0 : 1;
-                u.w[0] = u.w[1 - done] - u.w[done];
-                u.n = 1;
-            } else {
-                u.n = 0;
-            }
-            u.t = ev.first;
-            end = ev.first > end ? ev.first : end;
-            if (next < jobs.size()) u.w[u.n++] = jobs[next++];
-            if (u.n) heap.push(Ev(event(u), ev.second));
-        }
-        return end;
-    };
-    size_t chunk = (size_t)longest;
-    double best = simulate(longest);
-    for (int k = 2; k <= 64 && k <= longest; k++) {
-        const int c = (longest + k - 1) / k;
-        if ((size_t)c >= chunk) continue;
-        // more than eight pieces per CU never measured faster; the bound
-        // also keeps the simulation to a few thousand pieces
-        size_t n = 0;
-        for (int nb : nbs) n += (size_t)((nb + c - 1) / c);
-        if (n * p.groups > 8 * cus) break;   // smaller chunks only add pieces
-        const double e = simulate(c);
-        if (e < best - 1e-9) {
-            best = e;
-            chunk = (size_t)c;
-        }
-    }
-    const int ovr = tuning_env(TUNE_ATTN_MFMA_SPLIT);   // pieces of the longest query block (tuning)
-    if (ovr > 0) chunk = ((size_t)longest + (size_t)ovr - 1) / (size_t)ovr;
-    if (chunk < 1) chunk = 1;
-    if (chunk >= (size_t)longest) return p;   // every query block in one piece
-    const size_t nbmax = (kv_len + 31) / 32;
-    p.chunk = (int)chunk;
-    p.stride = (int)((nbmax + chunk - 1) / chunk);
-    return p;
-}
-
-static int cu_count_attn() {
+int cu_count_attn() {
     static std::atomic<int> n[64] = {};   // per device; racing callers store the same value
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
@@ -932,10 +521,7 @@ static int cu_count_attn() {
 }
 
 size_t attention_workspace(size_t n_head, size_t head_dim, size_t q_len, size_t kv_len, size_t n_head_kv) {
-    if (head_dim == 128 && q_len >= (size_t)attn_mfma_min_q() && kv_len < ((size_t)1 << 23)) {
-        const AmPlan p = attn_mfma_plan(n_head, n_head_kv, q_len, kv_len);
-        return p.chunk > 0 ? (size_t)p.stride * n_head * q_len * (head_dim + 2) * sizeof(float) : 0;
-    }
+    if (attn_prompt_path(n_head, n_head_kv, head_dim, q_len, kv_len)) return attn_prompt_workspace(n_head, n_head_kv, head_dim, q_len, kv_len);
     int ns = 0, chunk = 0;
     attention_plan(n_head, n_head_kv, q_len, kv_len, &ns, &chunk);
     return ns > 1 ? (size_t)ns * n_head * q_len * (head_dim + 2) * sizeof(float) : 0;
@@ -979,7 +565,7 @@ void attention_plan(size_t n_head, size_t n_head_kv, size_t q_len, size_t kv_len
 // quantizes them.
 bool attention_q8_direct(const AttnArgs& a) {
     if ((a.n_head * a.head_dim) % 256 != 0) return false;
-    if (attn_mfma_path(a)) return attn_mfma_plan(a.n_head, a.n_head_kv, a.q_len, a.kv_len).chunk > 0;
+    if (attn_prompt_path(a.n_head, a.n_head_kv, a.head_dim, a.q_len, a.kv_len)) return attn_prompt_q8_direct(a);
     int ns = 0, chunk = 0;
     attention_plan(a.n_head, a.n_head_kv, a.q_len, a.kv_len, &ns, &chunk);
     return ns > 1;
@@ -1017,39 +603,7 @@ static hipError_t attn_launch_hd(const AttnArgs& a, hipStream_t s) {
 
 hipError_t attention_launch(const AttnArgs& a, hipStream_t s) {
     if (a.q_len == 0 || a.n_head == 0) return hipSuccess;
-    if (attn_mfma_path(a)) {
-        const float scale = (1.0f / sqrtf(128.0f)) * LOG2E;
-        const AmPlan p = attn_mfma_plan(a.n_head, a.n_head_kv, a.q_len, a.kv_len);
-        const int w = p.w;
-        const bool pair = p.pair;
-        unsigned nx = pair ? (p.nqb + 1) / 2 : p.nqb;
-        if (p.chunk > 0) {   // the pieces of every query block at the actual start position
-            nx = 0;
-            for (unsigned qb = 0; qb < p.nqb; qb++)
-                nx += (unsigned)((am_qblock_blocks((int)qb, (int)a.q_len, (int)a.kv_len, (long long)a.start_pos) +
-                                  p.chunk - 1) / p.chunk);
-        }
-        const dim3 grid = p.chunk > 0 ? dim3(nx * p.groups, 1, 1) : dim3(nx, p.groups, 1);
-#define BARQ_AM_LAUNCH(W_, P_)                                                                                    \
-    hipLaunchKernelGGL((attn_mfma_kernel<W_, P_>), grid, dim3(64 * W_), 0, s, a.q, a.k, a.v, a.layer_off,           \
-                       a.head_stride, (int)a.n_head, (int)a.n_head_kv, (int)a.q_len, (int)a.kv_len,               \
-                       (long long)a.start_pos, scale, a.out, a.part, p.chunk, p.stride)
-        if (w == 4) { if (pair) BARQ_AM_LAUNCH(4, true); else BARQ_AM_LAUNCH(4, false); }
-        else if (w == 2) { if (pair) BARQ_AM_LAUNCH(2, true); else BARQ_AM_LAUNCH(2, false); }
-        else { if (pair) BARQ_AM_LAUNCH(1, true); else BARQ_AM_LAUNCH(1, false); }
-#undef BARQ_AM_LAUNCH
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess || p.chunk == 0) return e;
-        // (the plan splits only when the rows are whole Q8_K blocks)
-        const dim3 cg((unsigned)(a.n_head * 128 / 256), (unsigned)a.q_len);
-        if (a.out_q8)
-            hipLaunchKernelGGL((attn_combine_few_kernel<128, true>), cg, dim3(256), 0, s, a.part, p.stride, p.chunk,
-                               (int)a.n_head, (int)a.q_len, (int)a.kv_len, (long long)a.start_pos, a.out, a.out_q8);
-        else
-            hipLaunchKernelGGL((attn_combine_few_kernel<128, false>), cg, dim3(256), 0, s, a.part, p.stride, p.chunk,
-                               (int)a.n_head, (int)a.q_len, (int)a.kv_len, (long long)a.start_pos, a.out, a.out_q8);
-        return hipGetLastError();
-    }
+    if (attn_prompt_path(a.n_head, a.n_head_kv, a.head_dim, a.q_len, a.kv_len)) return attn_prompt_launch(a, s);
     switch (a.head_dim) {
     case 64: return attn_launch_hd<64>(a, s);
     case 128: return attn_launch_hd<128>(a, s);

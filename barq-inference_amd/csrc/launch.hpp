@@ -200,5 +200,12 @@ hipError_t stream_read_launch(const void* p, size_t bytes, uint32_t* sink, hipSt
 void attention_plan(size_t n_head, size_t n_head_kv, size_t q_len, size_t kv_len, int* n_split, int* chunk);
 size_t attention_workspace(size_t n_head, size_t head_dim, size_t q_len, size_t kv_len, size_t n_head_kv);
 hipError_t attention_launch(const AttnArgs& a, hipStream_t s);
+int cu_count_attn();   // CUs of the current device
+
+// attention_prompt.hip: chunks of many query rows on the matrix cores
+bool attn_prompt_path(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len);
+size_t attn_prompt_workspace(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len);
+bool attn_prompt_q8_direct(const AttnArgs& a);
+hipError_t attn_prompt_launch(const AttnArgs& a, hipStream_t s);
 
 }  // namespace barq

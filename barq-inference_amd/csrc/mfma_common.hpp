@@ -37,10 +37,13 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // wait-count insertion does not treat every in-flight stage as a pending
 // write to the stage being read (it would drain them all); the kernels wait
 // on their own loads with wait_vmcnt before each barrier.
-__device__ __forceinline__ void lds_load16(i32x4v r, void* lds_wave_base, uint32_t voff, uint32_t soff) {
-    const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_addr(lds_wave_base));
+__device__ __forceinline__ void lds_load16_at(i32x4v r, uint32_t lds_wave_addr, uint32_t voff, uint32_t soff) {
+    const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds_wave_addr);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :: "s"(m0), "v"(voff), "s"(r), "s"(soff) : "memory", "m0");
+}
+__device__ __forceinline__ void lds_load16(i32x4v r, void* lds_wave_base, uint32_t voff, uint32_t soff) {
+    lds_load16_at(r, lds_addr(lds_wave_base), voff, soff);
 }
 // The same with the non-temporal hint (`nt`), for the streamed GEMV weight
 // slices: measured on MI355X in one run, the 128256 x 4096 Q6_K GEMV 72.5 ->

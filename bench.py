@@ -973,8 +973,8 @@ def bench_attn(args):
         t_cpu = time.perf_counter() - t0
     err = float(np.max(np.abs(got - ref)) / np.max(np.abs(vh)))
     cpu_gbs = alg * calls / t_cpu / 1e9
-    # prompt chunks of 32+ rows run the f32-MFMA kernel: compute-bound
-    mfma = ql >= int(os.environ.get("BARQ_ATTN_MFMA_MIN_Q", "32"))
+    # prompt chunks run the MFMA kernel (from about 200 rows at position 0): compute-bound
+    mfma = ql >= int(os.environ.get("BARQ_ATTN_MFMA_MIN_Q", "200"))
     tflops = flops / (ms * 1e-3) / 1e12
     if mfma:
         roof = {"bound": "mfma", "achieved": round(tflops, 2), "peak": F32_MFMA_PEAK_TFLOPS, "unit": "TFLOP/s (f32)",
