@@ -1,0 +1,43 @@
+"""Tile choices of the batched GEMMs that depend on how many tiles a shape has."""
+import os
+
+import numpy as np
+import pytest
+
+import barq_rocm as B
+from barq_rocm import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def backend(**env):
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update(env)
+    try:
+        return B.Backend(0)
+    finally:
+        for k, v in old.items():
+            os.environ.pop(k) if v is None else os.environ.__setitem__(k, v)
+
+
+@pytest.mark.parametrize("rows", [41, 63, 64, 65, 129])
+def test_expert_groups_of_64_row_tiles(be, rows):
+    """Expert groups above 40 rows take 64-row tiles; a weight row's products
+    are summed in the same order as on 32-row tiles, so the outputs are the
+    same bits.  Three experts with `rows` - 20, `rows` and `rows` + 20 rows."""
+    hidden, n_ff, ne = 512, 768, 3
+    g, u = ([dev(synth.gen_q4_k(n_ff, hidden, 10 * e + s)) for e in range(ne)] for s in (1, 2))
+    d = [dev(synth.gen_q6_k(hidden, n_ff, 10 * e + 3)) for e in range(ne)]
+    ids = np.concatenate([np.full(rows + 20 * (e - 1), e) for e in range(ne)]).astype(np.int32)
+    ids = np.random.default_rng(rows).permutation(ids)[:, None]
+    x, w = synth.gen_f32(len(ids) * hidden, 5).reshape(-1, hidden), np.ones((len(ids), 1), np.float32)
+    small = backend(BARQ_GEMM_BM="32")
+    outs = [b.moe_ffn(B.Q4_K, g, B.Q4_K, u, B.Q6_K, d, hidden, n_ff, dev(x), len(ids), dev(ids), dev(w), 1,
+                      B.ACT_F32_Q8).cpu().numpy() for b in (be, small)]
+    small.close()
+    assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
