@@ -9,12 +9,20 @@
 // 32x32 tile of one block's exact integer dot products, which the epilogue
 // scales by dx * dw in f32.  Unlike the K-quant kernel (gemm_kq.hip), the
 // per-block scales are floats, so they cannot be folded into the int8
-// operands; the f32 epilogue (three vector instructions per output element
-// per block) is what bounds this kernel.
+// operands, and the f32 epilogue is what bounds this kernel.  The scales are
+// f16 (GGUF formats), so their products are exact in f32, and a second MFMA
+// (f16, one of its 16 k slots used) forms the tile's dx * dw: two vector
+// instructions per output element per block are left (conversion, fma)
+// instead of three, and a lane reads one activation scale per tile and block
+// from LDS instead of sixteen.  The same bits as dx * dw on the vector units.
+// Measured on MI355X, us per call, before / after, same tiles: Q8_0 4096 x
+// 4096, M = 512 46.1 / 41.7; Q4_0 14336 x 4096, M = 512 146 / 132; Q8_0 9000 x
+// 5120, M = 700 189 / 165.
 //
 // The Q8_0 activation rows are first repacked (q8_0_repack_kernel) into
 // plain int8 rows (16-byte aligned blocks) and a table of the block scales
-// as f32 in [block][row] order.  Per workgroup: BM activation rows x 128
+// in [block][row] order, as f16 bits (as f32 for the quant crate's Q4_0,
+// whose weight scales are f32).  Per workgroup: BM activation rows x 128
 // weight rows; four waves, each 32 weight rows and all BM activation rows.
 // A step is four blocks (128 elements): NS LDS stages, each filled by
 // buffer->LDS loads NS-1 steps ahead with one barrier per step (as in
@@ -27,18 +35,20 @@
 namespace barq {
 
 // ---- activation repack ---------------------------------------------------------
-// Q8_0 block b of row r -> 32 int8 at xr[r * k + 32 b], f32 scale at dx[b * m + r].
+// Q8_0 block b of row r -> 32 int8 at xr[r * k + 32 b], scale at dx[b * m + r]
+// (f16 bits in the low half, or f32 with F32).
 // A workgroup takes 16 rows x 16 blocks: thread t reads block t % 16 of row
 // t / 16 (each row's blocks contiguous), and the scales go out through LDS as
 // 16 runs of 16 consecutive rows.
+template <bool F32>
 __global__ __launch_bounds__(256) void q8_0_repack_kernel(const uint8_t* __restrict__ xq, size_t m, size_t nblk,
-                                                          int8_t* __restrict__ xr, float* __restrict__ dx) {
-    __shared__ float sd[16][17];
+                                                          int8_t* __restrict__ xr, uint32_t* __restrict__ dx) {
+    __shared__ uint32_t sd[16][17];
     const int t = threadIdx.x;
     const size_t r = (size_t)blockIdx.y * 16 + t / 16, b = (size_t)blockIdx.x * 16 + (t & 15);
     if (r < m && b < nblk) {
         const uint8_t* blk = xq + (r * nblk + b) * Q8_0_BYTES;
-        sd[t & 15][t / 16] = f16_bits_to_f32(ld_u16(blk));
+        sd[t & 15][t / 16] = F32 ? __builtin_bit_cast(uint32_t, f16_bits_to_f32(ld_u16(blk))) : ld_u16(blk);
         uint4* dst = reinterpret_cast<uint4*>(xr + (r * nblk + b) * 32);
         dst[0] = ld16_a2(blk + 2);
         dst[1] = ld16_a2(blk + 18);
@@ -70,10 +80,13 @@ __device__ __forceinline__ uint4 lds_u4(const uint8_t* base) {
 }
 
 template <int OFF>
-__device__ __forceinline__ float lds_f16(const uint8_t* base) {
+__device__ __forceinline__ uint32_t lds_u16(const uint8_t* base) {
     const uint32_t w = *reinterpret_cast<const uint32_t*>(base + (OFF & ~3));
-    return f16_bits_to_f32((OFF & 2) ? w >> 16 : w & 0xFFFFu);
+    return (OFF & 2) ? w >> 16 : w & 0xFFFFu;
 }
+
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // q - 8 for four nibbles q in [0, 15] (one per byte): no byte carries.
 __device__ __forceinline__ uint32_t nib_minus8(uint32_t q) { return (q + 0x78787878u) ^ 0x80808080u; }
@@ -82,24 +95,26 @@ __device__ __forceinline__ uint32_t nib_minus8(uint32_t q) { return (q + 0x78787
 // low nibble of qs[i], element i + 16 the high nibble; value (q - 8) * d.
 struct B40 {
     static constexpr int TYPE = TYPE_Q4_0, BB = Q4_0_BYTES, WP = 5, PIECES = 5, SHIFT = 8, NS = 3, KG_MAX = 4;
+    static constexpr bool F16_SCALE = true;
     template <int J>
-    static __device__ __forceinline__ void block(const uint8_t* row, int g2, v4i& b, float& dw) {
+    static __device__ __forceinline__ void block(const uint8_t* row, int g2, v4i& b, uint32_t& dw) {
         const uint4 qs = lds_u4<18 * J + 2>(row);
         const uint32_t sh = 4u * (uint32_t)g2;
         b = v4i{(int)nib_minus8((qs.x >> sh) & 0x0F0F0F0Fu), (int)nib_minus8((qs.y >> sh) & 0x0F0F0F0Fu),
                 (int)nib_minus8((qs.z >> sh) & 0x0F0F0F0Fu), (int)nib_minus8((qs.w >> sh) & 0x0F0F0F0Fu)};
-        dw = lds_f16<18 * J>(row);
+        dw = lds_u16<18 * J>(row);
     }
 };
 
 // GGUF Q8_0 (gguf.rs:634-681): f16 d + 32 int8.
 struct B80 {
     static constexpr int TYPE = TYPE_Q8_0, BB = Q8_0_BYTES, WP = 9, PIECES = 9, SHIFT = 8, NS = 2, KG_MAX = 2;
+    static constexpr bool F16_SCALE = true;
     template <int J>
-    static __device__ __forceinline__ void block(const uint8_t* row, int g2, v4i& b, float& dw) {
+    static __device__ __forceinline__ void block(const uint8_t* row, int g2, v4i& b, uint32_t& dw) {
         const uint4 q = lds_u4<34 * J + 2>(row + 16 * g2);   // quants 16 g2 .. 16 g2 + 15
         b = v4i{(int)q.x, (int)q.y, (int)q.z, (int)q.w};
-        dw = lds_f16<34 * J>(row);
+        dw = lds_u16<34 * J>(row);
     }
 };
 
@@ -107,12 +122,13 @@ struct B80 {
 // (low nibble for even i), value (nib >= 8 ? nib - 16 : nib) * scale.
 struct B40Barq {
     static constexpr int TYPE = TYPE_Q4_0_BARQ, BB = Q4_0_BARQ_BYTES, WP = 5, PIECES = 5, SHIFT = 0, NS = 3, KG_MAX = 4;
+    static constexpr bool F16_SCALE = false;
     // four nibbles (even or odd elements) -> signed bytes: (nib ^ 8) - 8
     static __device__ __forceinline__ uint32_t sext4(uint32_t v) {
         return ((v ^ 0x08080808u) + 0x78787878u) ^ 0x80808080u;
     }
     template <int J>
-    static __device__ __forceinline__ void block(const uint8_t* row, int g2, v4i& b, float& dw) {
+    static __device__ __forceinline__ void block(const uint8_t* row, int g2, v4i& b, uint32_t& dw) {
         // elements 16 g2 .. 16 g2 + 15 are bytes 8 g2 .. 8 g2 + 7 of the 16 quant bytes
         const uint32_t* q = reinterpret_cast<const uint32_t*>(row + 20 * J + 4 + 8 * g2);
         const uint32_t d0 = q[0], d1 = q[1];
@@ -121,7 +137,7 @@ struct B40Barq {
         // interleave even (lo) and odd (hi) elements back into element order
         b = v4i{(int)__builtin_amdgcn_perm(hi0, lo0, 0x05010400u), (int)__builtin_amdgcn_perm(hi0, lo0, 0x07030602u),
                 (int)__builtin_amdgcn_perm(hi1, lo1, 0x05010400u), (int)__builtin_amdgcn_perm(hi1, lo1, 0x07030602u)};
-        dw = *reinterpret_cast<const float*>(row + 20 * J);
+        dw = *reinterpret_cast<const uint32_t*>(row + 20 * J);
     }
 };
 
@@ -194,21 +210,33 @@ __device__ __forceinline__ void b32_block(const uint8_t* st, const uint8_t* wrow
     using L = B32L<F, BM>;
     constexpr int MT = L::MT;
     v4i b;
-    float dw;
+    uint32_t dw;   // the weight block's scale: f16 bits, or f32 ones
     F::template block<J>(wrow, g2, b, dw);
+    // k slot 0 of lane half 0 carries the scales; every other slot is 0 * 0
+    const h8v bs = __builtin_bit_cast(h8v, v4i{g2 ? 0 : (int)dw, 0, 0, 0});
     #pragma unroll
     for (int t = 0; t < MT; t++) {
         const v4i a = *reinterpret_cast<const v4i*>(st + (mbase + 32 * t + n) * B32_XRS + 32 * J + 16 * g2);
         const v16i z = {};
         const v16i c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, z, 0, 0, 0);
-        #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            // rows 32t + 8q + 4g2 .. +3 of the wave's rows (32x32 C layout)
-            const float4 dx = *reinterpret_cast<const float4*>(st + L::DX + 4 * (J * BM + mbase + 32 * t + 8 * q + 4 * g2));
-            acc[t][4 * q + 0] = __builtin_fmaf(dx.x * dw, (float)c[4 * q + 0], acc[t][4 * q + 0]);
-            acc[t][4 * q + 1] = __builtin_fmaf(dx.y * dw, (float)c[4 * q + 1], acc[t][4 * q + 1]);
-            acc[t][4 * q + 2] = __builtin_fmaf(dx.z * dw, (float)c[4 * q + 2], acc[t][4 * q + 2]);
-            acc[t][4 * q + 3] = __builtin_fmaf(dx.w * dw, (float)c[4 * q + 3], acc[t][4 * q + 3]);
+        if constexpr (F::F16_SCALE) {
+            const int dx = *reinterpret_cast<const int*>(st + L::DX + 4 * (J * BM + mbase + 32 * t + n));
+            const f32x16 zf = {};
+            const f32x16 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8v, v4i{g2 ? 0 : dx, 0, 0, 0}), bs,
+                                                                    zf, 0, 0, 0);
+            #pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] = __builtin_fmaf(s[r], (float)c[r], acc[t][r]);
+        } else {
+            const float dwf = __builtin_bit_cast(float, dw);
+            #pragma unroll
+            for (int q = 0; q < 4; q++) {
+                // rows 32t + 8q + 4g2 .. +3 of the wave's rows (32x32 C layout)
+                const float4 dx = *reinterpret_cast<const float4*>(st + L::DX + 4 * (J * BM + mbase + 32 * t + 8 * q + 4 * g2));
+                acc[t][4 * q + 0] = __builtin_fmaf(dx.x * dwf, (float)c[4 * q + 0], acc[t][4 * q + 0]);
+                acc[t][4 * q + 1] = __builtin_fmaf(dx.y * dwf, (float)c[4 * q + 1], acc[t][4 * q + 1]);
+                acc[t][4 * q + 2] = __builtin_fmaf(dx.z * dwf, (float)c[4 * q + 2], acc[t][4 * q + 2]);
+                acc[t][4 * q + 3] = __builtin_fmaf(dx.w * dwf, (float)c[4 * q + 3], acc[t][4 * q + 3]);
+            }
         }
     }
 }
@@ -236,7 +264,7 @@ __device__ __forceinline__ void b32_compute(const uint8_t* st, int s, int wave, 
 template <class F, int BM, int NS, int KG>
 __global__ __launch_bounds__(256 * KG, 1)
 void b32_gemm_kernel(const uint8_t* __restrict__ W, uint32_t wrb, const int8_t* __restrict__ X,
-                     const float* __restrict__ DXT, float* __restrict__ Y, int M, int N, int K, int tiles_m,
+                     const uint32_t* __restrict__ DXT, float* __restrict__ Y, int M, int N, int K, int tiles_m,
                      int ks, int xcd_order) {
     using L = B32L<F, BM>;
     constexpr int MT = L::MT, SB = KG * L::STAGE;
@@ -267,11 +295,20 @@ void b32_gemm_kernel(const uint8_t* __restrict__ W, uint32_t wrb, const int8_t* 
     const int s0 = slice * nst * KG;                // this slice's first step
     const int sub = kg * L::STAGE;
 
-    float acc[MT][16];
+    // With one K-group the two halves of K have sums of their own, added at the
+    // end: chains no longer than with two K-groups (error against 64 bits at k =
+    // 4096 1.5e-7, one chain 2.0e-7).
+    float acc[MT][16], half[KG == 1 ? MT : 1][16];
     #pragma unroll
     for (int t = 0; t < MT; t++)
         #pragma unroll
         for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+    if constexpr (KG == 1) {
+        #pragma unroll
+        for (int t = 0; t < MT; t++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++) half[t][r] = 0.0f;
+    }
 
     #pragma unroll
     for (int s = 0; s < NS - 1; s++)
@@ -292,6 +329,23 @@ void b32_gemm_kernel(const uint8_t* __restrict__ W, uint32_t wrb, const int8_t* 
         if (s + NS - 1 < nst)
             b32_issue<F, BM>(stage((s + NS - 1) % NS) + sub, xr, wr, dr, off, s0 + KG * (s + NS - 1) + kg, m, wave);
         b32_compute<F, BM>(stage(s % NS) + sub, s0 + KG * s + kg, wave, l, acc);
+        if constexpr (KG == 1) {
+            if (s + 1 == nst / 2) {
+                #pragma unroll
+                for (int t = 0; t < MT; t++)
+                    #pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        half[t][r] = acc[t][r];
+                        acc[t][r] = 0.0f;
+                    }
+            }
+        }
+    }
+    if constexpr (KG == 1) {
+        #pragma unroll
+        for (int t = 0; t < MT; t++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] += half[t][r];
     }
 
     if constexpr (KG > 1) {
@@ -345,7 +399,7 @@ __global__ __launch_bounds__(256) void slice_sum_kernel(const float* __restrict_
 // ---- launch ------------------------------------------------------------------
 
 template <class F, int BM, int NS, int KG>
-static hipError_t b32_launch_t(const void* W, size_t n_rows, size_t k, const int8_t* xr, const float* dx, size_t m,
+static hipError_t b32_launch_t(const void* W, size_t n_rows, size_t k, const int8_t* xr, const uint32_t* dx, size_t m,
                                float* y, int ks, hipStream_t s) {
     const int tiles_m = (int)((m + BM - 1) / BM), tiles_n = (int)((n_rows + B32_BN - 1) / B32_BN);
     const uint32_t wrb = (uint32_t)(k / 32 * F::BB);
@@ -356,8 +410,23 @@ static hipError_t b32_launch_t(const void* W, size_t n_rows, size_t k, const int
     return hipGetLastError();
 }
 
-static int b32_bm(size_t m) {
-    const int bm = tuning_env(TUNE_GEMM_BM, m > 32 ? 64 : 32);
+// More 64-row tiles than CUs: one K-group of four waves per workgroup, so that
+// two or three workgroups share a CU and a last round that leaves CUs without
+// a tile costs less; fewer than two tiles per CU are cut into 32-row ones.
+// Measured on MI355X, us per call with the repack, for 64-row tiles with two
+// K-groups (one workgroup per CU) / 64-row / 32-row tiles with one, two
+// stages each: Q8_0 6144 x 4096, M = 333 (288 tiles, f32 rows) 70.9 / 62.3 /
+// 58.8; Q4_0 the same 66.5 / 54.1 / 48.9; Q4_0 14336 x 4096, M = 512 (896)
+// 131 / 99 / 107 (118 / 125 with three stages, which leave room for two
+// workgroups instead of three); Q4_0 9000 x 5120, M = 700 (781) 166 / 122 /
+// 137; with a tile per CU (Q4_0 4096 x 4096, M = 512) 38.0 / 45.7 / 40.1.
+static bool b32_many_tiles(size_t m, size_t n_rows) {
+    return (m + 63) / 64 * ((n_rows + B32_BN - 1) / B32_BN) > 256;
+}
+
+static int b32_bm(size_t m, size_t n_rows) {
+    const bool few = b32_many_tiles(m, n_rows) && (m + 63) / 64 * ((n_rows + B32_BN - 1) / B32_BN) < 512;
+    const int bm = tuning_env(TUNE_GEMM_BM, m > 32 && !few ? 64 : 32);
     return bm == 32 ? 32 : 64;
 }
 
@@ -365,7 +434,7 @@ static int b32_bm(size_t m) {
 // doubled while the grid stays within 256 workgroups and every slice keeps
 // an even number of steps.  BARQ_GEMM_KS overrides.
 static int b32_k_slices(size_t m, size_t n_rows, size_t k) {
-    const int bm = b32_bm(m);
+    const int bm = b32_bm(m, n_rows);
     const size_t tiles = (m + bm - 1) / bm * ((n_rows + B32_BN - 1) / B32_BN), steps = k / (32 * B32_SB);
     int ks = 1;
     while (ks < 16 && tiles * ks * 2 <= 256 && steps % (size_t)(ks * 4) == 0) ks *= 2;
@@ -374,22 +443,22 @@ static int b32_k_slices(size_t m, size_t n_rows, size_t k) {
     return ks;
 }
 
-// Tile rows and K-groups: 64-row tiles above 32 rows; four K-groups when
-// there are fewer tiles than CUs and the step count allows, else two (two
-// with K slices).  BARQ_GEMM_BM (32, 64) and BARQ_GEMM_KG (1, 2, 4) override.
+// Tile rows and K-groups: 64-row tiles above 32 rows; one K-group with more
+// tiles than CUs (b32_many_tiles); four when there are fewer and the step
+// count allows, else two (two with K slices).  BARQ_GEMM_BM (32, 64) and BARQ_GEMM_KG (1, 2, 4) override.
 template <class F>
-static hipError_t b32_dispatch(const void* W, size_t n_rows, size_t k, const int8_t* xr, const float* dx, size_t m,
+static hipError_t b32_dispatch(const void* W, size_t n_rows, size_t k, const int8_t* xr, const uint32_t* dx, size_t m,
                                float* y, int ks, hipStream_t s) {
-    const int bm = b32_bm(m);
+    const int bm = b32_bm(m, n_rows);
     const size_t tiles = (m + bm - 1) / bm * ((n_rows + B32_BN - 1) / B32_BN);
     const size_t steps = k / (32 * B32_SB) / ks;   // per slice
-    int kg = tuning_env(TUNE_GEMM_KG, ks == 1 && tiles < 256 && steps % 4 == 0 ? 4 : 2);
+    int kg = tuning_env(TUNE_GEMM_KG, b32_many_tiles(m, n_rows) ? 1 : ks == 1 && tiles < 256 && steps % 4 == 0 ? 4 : 2);
     if (kg != 1 && kg != 2 && kg != 4) kg = 2;
     if (kg > F::KG_MAX) kg = F::KG_MAX;   // LDS: Q8_0 weight rows are twice as long
     if (steps % kg != 0) kg = steps % 2 == 0 ? 2 : 1;
 #define B32_CASE(BMV, KGV) \
     if constexpr (KGV <= F::KG_MAX) \
-        if (bm == BMV && kg == KGV) return b32_launch_t<F, BMV, (KGV == 4 ? 2 : F::NS), KGV>(W, n_rows, k, xr, dx, m, y, ks, s);
+        if (bm == BMV && kg == KGV) return b32_launch_t<F, BMV, (KGV != 2 ? 2 : F::NS), KGV>(W, n_rows, k, xr, dx, m, y, ks, s);
     B32_CASE(32, 1) B32_CASE(32, 2) B32_CASE(32, 4) B32_CASE(64, 1) B32_CASE(64, 2) B32_CASE(64, 4)
 #undef B32_CASE
     return b32_launch_t<F, 64, F::NS, 2>(W, n_rows, k, xr, dx, m, y, ks, s);
@@ -416,8 +485,9 @@ hipError_t b32_gemm_launch(int w_type, const void* W, size_t n_rows, size_t k, c
     if (!b32_supported(w_type, n_rows, k, m)) return hipErrorInvalidValue;
     const size_t nblk = k / 32;
     int8_t* xr = static_cast<int8_t*>(ws);
-    float* dx = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + m * k);
-    hipLaunchKernelGGL(q8_0_repack_kernel, dim3((unsigned)((nblk + 15) / 16), (unsigned)((m + 15) / 16)), dim3(256), 0, s,
+    uint32_t* dx = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(ws) + m * k);
+    auto* repack = w_type == TYPE_Q4_0_BARQ ? &q8_0_repack_kernel<true> : &q8_0_repack_kernel<false>;
+    hipLaunchKernelGGL(repack, dim3((unsigned)((nblk + 15) / 16), (unsigned)((m + 15) / 16)), dim3(256), 0, s,
                        static_cast<const uint8_t*>(xq), m, nblk, xr, dx);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -41,3 +41,22 @@ def test_expert_groups_of_64_row_tiles(be, rows):
                       B.ACT_F32_Q8).cpu().numpy() for b in (be, small)]
     small.close()
     assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("t", [B.Q4_0, B.Q8_0, B.Q4_0_BARQ])
+@pytest.mark.parametrize("n,m,scale", [
+    (16400, 65, 1.0),     # 258 tiles of 64 rows: 32-row tiles, one K-group
+    (21800, 130, 1.0),    # 513 tiles: 64-row tiles, one K-group
+    (200, 70, 1e-6),      # activation scales that are subnormal in f16
+    (200, 33, 3e4),       # large ones
+])
+def test_32_element_blocks_many_tiles(be, orc, t, n, m, scale):
+    """Against the oracle at 1e-6: integer products are exact, the f16 scales'
+    products too, and k / 32 = 8 terms are summed in f32."""
+    k = 256
+    w, x = synth.gen_weights(t, n, k, 7), synth.gen_f32(m * k, 8).reshape(m, k) * np.float32(scale)
+    xq = be.quantize_act(B.Q8_0, dev(x))
+    y = be.matmul(t, dev(w), n, k, B.Q8_0, xq, m).cpu().numpy()
+    ref = orc.matmul(t, w, n, k, orc.Q8_0, xq.cpu().numpy(), m).reshape(m, n)
+    err = np.linalg.norm(y.astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64))
+    assert np.any(ref) and err <= 1e-6, err
