@@ -4,8 +4,8 @@
 
 namespace barq {
 
-// Overrides: BARQ_GEMM_BM (16, 32, 64, or 65 = 64 rows with eight waves of
-// 32 x 32 per K-group),
+// Overrides: BARQ_GEMM_BM (16, 32, 64, 65 = 64 rows with eight waves of
+// 32 x 32 per K-group, or for Q4_K 68 = 128 rows),
 // BARQ_GEMM_NS (stages), BARQ_GEMM_KG (K-groups, ungrouped), BARQ_GEMM_KS
 // (K slices: the MoE down projection, and ungrouped launches).
 
@@ -37,6 +37,26 @@ static bool kq6_tall_tiles(size_t m, size_t n_rows, size_t nsb) {
     return m >= 256 && (nsb >= 32 || n_rows >= 8192);
 }
 
+// Q4_K prompts: 128 x 128 tiles of eight waves of 64 x 32, one K-group, two
+// stages.  The 64-row launch is bound by its buffer->LDS copies; a 128-row
+// tile copies each weight block for twice the rows (57 KB a step against 76
+// KB for the same products) with the same two waves per SIMD, and needs no
+// sum over K-groups.  A tile takes 1.75 to 2 times as long as a 64-row one (one
+// workgroup per CU either way), so it is chosen where the CUs then run at
+// most half as many rounds of tiles.  Measured on MI355X, us per call, 64-row
+// / 128-row tiles (rounds): 14336 x 4096, M = 512 95 / 91 (4 / 2), M = 256
+// 46.9 / 42.7 (2 / 1), M = 768 133 / 124 (6 / 3); 6144 x 4096, M = 512 42.9 /
+// 39.3 (2 / 1); 20000 x 4096, M = 100 44.4 / 38.1 (2 / 1); and where the rule
+// keeps 64 rows: 14336 x 4096, M = 333 70 / 79 (3 / 2); 20000 x 8192, M = 700
+// 302 / 311 (7 / 4); 9000 x 8192, M = 400 89 / 148 (2 / 2).
+static bool kq4_tall_tiles(size_t m, size_t n_rows) {
+    const int bm_env = tuning_env(TUNE_GEMM_BM);
+    if (bm_env) return bm_env == 68;
+    const size_t tiles_n = (n_rows + KQ_BN - 1) / KQ_BN, cus = (size_t)cu_count();
+    const auto rounds = [&](size_t bm) { return ((m + bm - 1) / bm * tiles_n + cus - 1) / cus; };
+    return rounds(64) >= 2 * rounds(128);
+}
+
 template <class F, bool GROUPED>
 static hipError_t kq_dispatch(const KQArgs& a, size_t rows, hipStream_t s) {
     // measured on MI355X: 64x128 tiles above 32 rows, 32-row tiles with four
@@ -62,6 +82,8 @@ static hipError_t kq_dispatch(const KQArgs& a, size_t rows, hipStream_t s) {
         // once for two MFMA row tiles), one K-group, three stages
         if (bm == 66) return kq_launch_t<F, 64, 3, 4, GROUPED>(a, s);
     }
+    if constexpr (!GROUPED && F::TYPE == TYPE_Q4_K)
+        if (kq4_tall_tiles(rows, (size_t)a.N)) return kq_launch_t<F, 128, 2, 8, GROUPED>(a, s);
     if constexpr (!GROUPED) {
         // two K-groups of waves share a tile's pipeline (twice the waves per
         // SIMD for the same LDS) when the super-block count is even

@@ -60,3 +60,20 @@ def test_32_element_blocks_many_tiles(be, orc, t, n, m, scale):
     ref = orc.matmul(t, w, n, k, orc.Q8_0, xq.cpu().numpy(), m).reshape(m, n)
     err = np.linalg.norm(y.astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64))
     assert np.any(ref) and err <= 1e-6, err
+
+
+@pytest.mark.parametrize("n,k,m", [
+    (16500, 256, 65),      # 258 tiles of 64 rows, 129 of 128: one round instead of two; ragged in both
+    (16512, 768, 128),     # whole tiles, an odd number of super-blocks
+    (11000, 512, 193),     # a last tile with one row in its upper half
+    (16500, 512, 129),     # 258 tiles of 128 rows too: 64-row tiles stay
+])
+def test_q4_k_prompts_on_128_row_tiles(be, orc, n, k, m):
+    """Against the oracle at 1e-6: a super-block's integer sums are exact and
+    up to three of them are added in f32."""
+    w, x = synth.gen_q4_k(n, k, 3), synth.gen_f32(m * k, 4).reshape(m, k)
+    xq = be.quantize_act(B.Q8_K, dev(x))
+    y = be.matmul(B.Q4_K, dev(w), n, k, B.Q8_K, xq, m).cpu().numpy()
+    ref = orc.matmul(B.Q4_K, w, n, k, orc.Q8_K, xq.cpu().numpy(), m).reshape(m, n)
+    err = np.linalg.norm(y.astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64))
+    assert np.any(ref) and err <= 1e-6, err
