@@ -346,14 +346,23 @@ __global__ __launch_bounds__(256) void moe_group_gather_q8k_kernel(
             tokens[p] = 0;
             wts[p] = 0.0f;
         }
-    const int b = blockIdx.x * 4 + wave;
-    if (b >= nb) return;   // whole waves
-    const int i = b / nbr, cb = b - i * nbr;
-    const int tok = i < total ? tokl[i] / k : 0;
-    const float4 v = reinterpret_cast<const float4*>(x + ((size_t)tok * nbr + cb) * 256)[lane];
-    const float vv[4] = {v.x, v.y, v.z, v.w};
-    q8_k_block(vv, lane, out + (size_t)b * 292);
+    for (int64_t b = (int64_t)blockIdx.x * 4 + wave; b < nb; b += (int64_t)gridDim.x * 4) {   // whole waves
+        const int i = (int)b / nbr, cb = (int)b - i * nbr;
+        const int tok = i < total ? tokl[i] / k : 0;
+        const float4 v = reinterpret_cast<const float4*>(x + ((size_t)tok * nbr + cb) * 256)[lane];
+        const float vv[4] = {v.x, v.y, v.z, v.w};
+        q8_k_block(vv, lane, out + (size_t)b * 292);
+    }
 }
+
+// Workgroups of the fused kernel: each groups all assignments before it
+// quantizes, so with many workgroups the grouping (three barriers per 256
+// assignments) costs more than the one block that each wave then quantizes.
+// At most this many, each wave striding over the blocks.  Measured on MI355X,
+// us per Mixtral-8x7B expert FFN of 512 tokens (16384 blocks) with at most
+// 256 / 512 / 1024 / 2048 workgroups and without a bound: 827 / 821 / 822 /
+// 821 / 834; 256 tokens 525 / 520 / 520 / 520 / 521.
+constexpr size_t MOE_GATHER_WGS = 1024;
 
 // BARQ_MOE_FUSED_GROUP=0 keeps grouping and gather-quantize in two launches
 int moe_fused_group_enabled() { return tuning_env(TUNE_MOE_FUSED_GROUP, 1); }
@@ -365,7 +374,8 @@ hipError_t moe_group_gather_q8k_launch(const int32_t* ids, const float* weights,
     if (n == 0 || n > (size_t)MOE_FUSED_MAX || n_experts == 0 || n_experts > (size_t)MOE_MAX_EXPERTS ||
         hidden % 256 != 0 || nb > (size_t)INT32_MAX)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(moe_group_gather_q8k_kernel, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, s, ids, weights,
+    const size_t wgs = (nb + 3) / 4 < MOE_GATHER_WGS ? (nb + 3) / 4 : MOE_GATHER_WGS;
+    hipLaunchKernelGGL(moe_group_gather_q8k_kernel, dim3((unsigned)wgs), dim3(256), 0, s, ids, weights,
                        (int)rows, (int)top_k, (int)n_experts, x, (int)nbr, static_cast<uint8_t*>(out), (int)nb, offsets,
                        tokens, wts, rowpos);
     return hipGetLastError();

@@ -77,3 +77,18 @@ def test_q4_k_prompts_on_128_row_tiles(be, orc, n, k, m):
     ref = orc.matmul(B.Q4_K, w, n, k, orc.Q8_K, xq.cpu().numpy(), m).reshape(m, n)
     err = np.linalg.norm(y.astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64))
     assert np.any(ref) and err <= 1e-6, err
+
+
+def test_expert_gather_of_more_blocks_than_workgroups(be):
+    """1031 assignments of 8 blocks (some experts out of range): each wave
+    quantizes several blocks, with the outputs of the two-launch form."""
+    hidden, n_ff, ne, n = 2048, 512, 3, 1031
+    g, u = ([dev(synth.gen_q4_k(n_ff, hidden, 10 * e + s)) for e in range(ne)] for s in (1, 2))
+    d = [dev(synth.gen_q6_k(hidden, n_ff, 10 * e + 3)) for e in range(ne)]
+    ids = np.random.default_rng(2).integers(-1, ne + 1, (n, 1)).astype(np.int32)
+    x, w = synth.gen_f32(n * hidden, 5).reshape(n, hidden), np.ones((n, 1), np.float32)
+    two = backend(BARQ_MOE_FUSED_GROUP="0")
+    outs = [b.moe_ffn(B.Q4_K, g, B.Q4_K, u, B.Q6_K, d, hidden, n_ff, dev(x), n, dev(ids), dev(w), 1,
+                      B.ACT_F32_Q8).cpu().numpy() for b in (be, two)]
+    two.close()
+    assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
