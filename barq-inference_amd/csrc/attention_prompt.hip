@@ -16,22 +16,28 @@
 // What bounds it.  v_mfma_f32_32x32x2_f32 has a sixteenth of the f16 matrix
 // rate (157 TFLOP/s against 2.5 PFLOP/s), and a kernel on it ran at 105
 // TFLOP/s.  Here every f32 operand x is scaled by a power of two and split
-// exactly as x = hi + lo + e into two f16 values, each rounded to nearest:
-// |e| <= 2^-24 |x|, f32's own rounding error, and a product takes three f16
-// MFMAs (hi hi, hi lo, lo hi; lo lo is below 2^-24 of it) with f32 sums, 5.3
-// times the f32 rate.  Scales keep the split away from f16's limits:
+// into two f16 values, each rounded to nearest: x = hi + lo + e with |e| <=
+// 2^-23 |x| (2^-25 root mean square; three quarters of all mantissas split
+// exactly), and a product takes three f16 MFMAs (hi hi, hi lo, lo hi; lo lo is
+// at most 2^-22 of it, 2^-24.6 root mean square) with f32 sums, 5.3 times the
+// f32 rate.  Scales keep the split away from f16's limits:
 //   K: per position, the row's largest |k| into [2^13, 2^14); the inverse
 //      multiplies the scores
 //   Q: per query row, the same
-//   P: probabilities times 2^2 (their exponents are then near 0, where f32 is
-//      finest); the running maximum is only moved when it grows by more than
-//      2^8, so p <= 2^10 and O is seldom rescaled
-//   V: per output dim, the block's largest |v| into [2^14, 2^15); the scale
+//   P: per query row and block, the largest p just below 2^15
+//   V: per output dim, the largest |v| so far into [2^14, 2^15); the scale
 //      only ever shrinks, and O's dim is multiplied by the ratio when it does
-// lo's spacing is 2^-24 below these scales, so elements down to 2^-14 of the
-// largest they share a scale with keep all 24 bits.  Infinities and NaN turn
-// into NaN here; a tile whose sums are not finite is computed again by
-// ap_rows_f32, on f32 MFMAs without scales.
+// f16 steps end at 2^-24.  K's and Q's elements below 2^-14 of the largest
+// they share a scale with therefore lose bits.  Weights and values spread
+// further (a first position that takes nearly all the weight; a large value
+// that a row does not see), and what they lose is not small against the
+// result when the large ones add little to it.  lo of P and V is held times
+// 2^11, so that its steps end at 2^-35: weights down to 2^-26 of their block's
+// largest (18 nats) and values down to 2^-25 keep all bits.  Weights further
+// down lose one per halving (in that block alone); a tile with values below
+// 2^-34 of their dim's scale, or with a scale that shrinks by more than that,
+// is computed again by ap_rows_f32, on f32 MFMAs without scales, and so is one
+// whose sums are not finite (infinities and NaN turn into NaN here).
 //
 // Data movement: a block's K and V rows are loaded into registers one block
 // ahead of the conversion, converted by all four waves and stored as f16 in
@@ -41,13 +47,11 @@
 //
 // Measured on MI355X, us per call with the merge (the f32-MFMA kernel for 128
 // dims, the decode kernel for 64, before this one): Llama-3-8B heads, 2048 /
-// 1024 / 512 / 256 tokens 170 / 60 / 35 / 23.5 against 322 / 133 / 55 / 31;
-// 200 rows after 800 with heads of 64 dims 24 against 49.  Error against 64
-// bits (relative 2-norm, both dims, 64 to 1000 rows, 0 to 5000 cached): 1.5e-7
-// to 2.8e-7 against 1.4e-7 to 4.6e-7.  The matrix unit is about a third busy:
-// a block is 48 MFMAs and some 280 vector instructions per wave, the shader
-// clock falls to about 1.7 GHz under both, and a software pipeline that put
-// every conversion beside MFMAs was not faster.
+// 1024 / 512 / 256 tokens 210 / 71 / 40 / 25.6 against 337 / 135 / 54 / 30;
+// 200 rows after 800 with heads of 64 dims 26 against 55.  (With lo as it is,
+// one scale per row for P and no look at V's spread: 190 / 68 / 37 / 24 / 25.
+// P V on f32 MFMAs: 317 / 100 / 48 / 27 / 28.)  Error against 64 bits (relative
+// 2-norm, the same calls) 1.6e-7 to 1.9e-7 against 2.0e-7 to 3.9e-7.
 #include "common.hpp"
 #include "launch.hpp"
 #include "mfma_common.hpp"
@@ -349,6 +353,26 @@ __device__ __forceinline__ void ap_split(float x0, float x1, float minus_one, ui
     lo = __builtin_bit_cast(uint32_t, r);
 }
 
+// x0, x1, given times 2^11 -> packed f16 (hi) and 2^11 times what hi leaves
+// (lo): lo's smallest step is then 2^-35 of x's unit instead of 2^-24.  Two
+// v_fma_mix{lo,hi}_f16 per value.
+struct ApExt {
+    float down, neg;   // 2^-11 and -2^11 in registers that the compiler knows nothing of
+};
+__device__ __forceinline__ ApExt ap_ext() {
+    ApExt e{0x1p-11f, -0x1p11f};
+    asm("" : "+s"(e.down), "+s"(e.neg));
+    return e;
+}
+__device__ __forceinline__ void ap_split_ext(float x0, float x1, const ApExt& e, uint32_t& hi, uint32_t& lo) {
+    const h2v h = {(_Float16)__builtin_fmaf(x0, e.down, 0.0f), (_Float16)__builtin_fmaf(x1, e.down, 0.0f)};
+    hi = __builtin_bit_cast(uint32_t, h);
+    asm("" : "+v"(hi));
+    const h2v g = __builtin_bit_cast(h2v, hi);
+    const h2v r = {(_Float16)__builtin_fmaf((float)g[0], e.neg, x0), (_Float16)__builtin_fmaf((float)g[1], e.neg, x1)};
+    lo = __builtin_bit_cast(uint32_t, r);
+}
+
 // The biased exponent of |x| (at least 15, so that the scales below are normal
 // f32 values; 255 for infinities) and the powers of two that take such an x
 // into [2^P, 2^(P + 1)) and back.
@@ -362,7 +386,8 @@ template <int P>
 __device__ __forceinline__ float ap_unscale(uint32_t e) { return __builtin_bit_cast(float, (e - P) << 23); }
 
 constexpr int AP_KQ = 13, AP_V = 14;
-constexpr float AP_P = 2.0f;
+constexpr int AP_P = 2;               // the largest p before its scale: its exponents are then near 0, where f32 is finest
+constexpr uint32_t AP_SPREAD = 34;    // octaves below a dim's largest |v| that the split takes
 
 template <int HD>
 struct ApRegs {
@@ -397,9 +422,10 @@ __device__ __forceinline__ void ap_vmax(uint8_t* lds, const ApRegs<HD>& r, int p
 }
 
 // The loaded block n as f16 hi and lo into its stage.  ve: the exponent state
-// of the thread's dim (0: nothing but zeros so far).
+// of the thread's dim (0: nothing but zeros so far).  bad: set when the thread's
+// values spread further than the split can hold.
 template <int HD>
-__device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, int n, int t, uint32_t& ve) {
+__device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, int n, int t, uint32_t& ve, bool& bad) {
     using L = ApLds<HD>;
     uint8_t* st = lds + (n & 1) * L::STAGE;
     const float mo = ap_minus_one();
@@ -428,25 +454,38 @@ __device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, in
         *reinterpret_cast<uint2*>(krow + L::KLO + 8 * L::TPR * i) = lo;
     }
     if (t % L::TPR == 0) reinterpret_cast<float*>(st + L::KF)[t / L::TPR] = ap_unscale<AP_KQ>(ke);
-    const uint32_t e = mx > 0.0f ? ap_exp(mx) : 0u;
+    uint32_t e = __builtin_bit_cast(uint32_t, mx) >> 23;
+    e = mx > 0.0f ? (e > 30u ? e : 30u) : 0u;
     float ratio = 1.0f;
     if (e > ve) {
         // (nothing to rescale while O's dim is zero)
         if (ve) {
             ratio = ve + 126u > e ? __builtin_bit_cast(float, (127u + ve - e) << 23) : 0.0f;
             reinterpret_cast<int*>(lds + L::GROW)[n & 1] = n;
+            bad |= e > ve + AP_SPREAD;
         }
         ve = e;
     }
-    const uint32_t vu = ve ? ve : 15u;
+    // The smallest of the thread's values that are not zero (2 |bits| - 1 orders
+    // them with zero last).  Dims below 2^-87 are left to the f32 kernel too.
+    // Standard normal values come that far apart once in 10^10.
+    uint32_t um = 0xFFFFFFFFu;
+    #pragma unroll
+    for (int j = 0; j < L::PP; j++) {
+        const uint32_t u = (__builtin_bit_cast(uint32_t, r.v[j]) << 1) - 1u;
+        um = u < um ? u : um;
+    }
+    bad |= um < (ve < 40u ? 0xFFFFFFFFu : (ve - AP_SPREAD) << 24);
+    const uint32_t vu = ve ? ve : 30u;
     if (part == 0) {
         reinterpret_cast<float*>(lds + L::VR)[HD * (n & 1) + d] = ratio;
         reinterpret_cast<float*>(lds + L::VS)[d] = ap_unscale<AP_V>(vu);
     }
-    const float vs = ap_scale<AP_V>(vu);
+    const float vs = ap_scale<AP_V + 11>(vu);
+    const ApExt ex = ap_ext();
     uint32_t hi[L::PP / 2], lo[L::PP / 2];
     #pragma unroll
-    for (int j = 0; j < L::PP / 2; j++) ap_split(r.v[2 * j] * vs, r.v[2 * j + 1] * vs, mo, hi[j], lo[j]);
+    for (int j = 0; j < L::PP / 2; j++) ap_split_ext(r.v[2 * j] * vs, r.v[2 * j + 1] * vs, ex, hi[j], lo[j]);
     // Positions 4 u .. 4 u + 3 of a row are 8 bytes at 32 s + 16 g + 8 w with
     // u = 4 s + 2 w + g: the 16 bytes (s, g) are those whose probabilities
     // lane half g holds for step s.
@@ -526,28 +565,34 @@ __device__ __forceinline__ void ap_compute(const uint8_t* lds, int n, int j0, co
         auto hb = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, bm), __builtin_bit_cast(int, bm), false, false);
         bm = fmaxf(__builtin_bit_cast(float, (int)hb[0]), __builtin_bit_cast(float, (int)hb[1])) * qf;
     }
-    if (__any(bm > m + 8.0f)) {
-        const float mn = fmaxf(m, bm);
+    // The block's reference is bi (its p at most 2^AP_P, the largest above half of
+    // that); o and lsum are relative to m.  Both are whole numbers, so their
+    // factors are exact powers of two; m follows the maximum when that has grown
+    // by 2^32.
+    const float bi = __builtin_ceilf(bm);
+    if (__any(bi > m + 32.0f)) {
+        const float mn = fmaxf(m, bi);
         const float corr = m == -INFINITY ? 0.0f : fast_exp2(m - mn);
         m = mn;
         lsum *= corr;
         #pragma unroll
         for (int t = 0; t < L::NB; t++) o[t] *= corr;
     }
-    // a row that has seen no position yet keeps m = -inf: its p are 0 against any reference
-    const float mref = m == -INFINITY ? 0.0f : m - AP_P;
-    const float mo = ap_minus_one();
+    const bool none = bi == -INFINITY;   // a row that sees no position of the block
+    const float pref = none ? 0.0f : bi - (float)AP_P, step = none ? 0.0f : fast_exp2(bi - (float)AP_P - m);
+    const float inv = step * (1.0f / (float)(1 << (15 - AP_P)));
+    const ApExt ex = ap_ext();
     float rs[8];
     uint32_t ph[8], pl[8];
     #pragma unroll
     for (int r = 0; r < 8; r++) {
-        const float p0 = fast_exp2(__builtin_fmaf(sc[2 * r], qf, -mref)), p1 = fast_exp2(__builtin_fmaf(sc[2 * r + 1], qf, -mref));
+        const float p0 = fast_exp2(__builtin_fmaf(sc[2 * r], qf, -pref)), p1 = fast_exp2(__builtin_fmaf(sc[2 * r + 1], qf, -pref));
         rs[r] = p0 + p1;
-        ap_split(p0, p1, mo, ph[r], pl[r]);
+        ap_split_ext(p0 * (float)(1 << (26 - AP_P)), p1 * (float)(1 << (26 - AP_P)), ex, ph[r], pl[r]);
     }
     // (as a tree: a chain of sixteen rounds more)
     const float rsum = ((rs[0] + rs[1]) + (rs[2] + rs[3])) + ((rs[4] + rs[5]) + (rs[6] + rs[7]));
-    lsum += swap32_add(rsum, rsum);   // + the other half-wave's positions
+    lsum = __builtin_fmaf(swap32_add(rsum, rsum), step, lsum);   // + the other half-wave's positions
     const uint8_t* vp = st + L::V + c * L::VRS + 16 * g;
     h8v bh[2], bl[2];
     #pragma unroll
@@ -555,23 +600,33 @@ __device__ __forceinline__ void ap_compute(const uint8_t* lds, int n, int j0, co
         bh[s] = __builtin_bit_cast(h8v, u32x4v{ph[4 * s], ph[4 * s + 1], ph[4 * s + 2], ph[4 * s + 3]});
         bl[s] = __builtin_bit_cast(h8v, u32x4v{pl[4 * s], pl[4 * s + 1], pl[4 * s + 2], pl[4 * s + 3]});
     }
-    // A block's products start from zero, the small ones first, and are added
-    // to O once: the matrix unit's f32 sums do not round to nearest, and over
-    // many blocks of one accumulator that adds up.
+    // A block's products start from zero and are added to O once: the matrix
+    // unit's f32 sums do not round to nearest, and over many blocks of one
+    // accumulator that adds up.
+    constexpr int U = HD == 64 ? 2 : 1;   // accumulators at a time (128 dims: two would not fit the registers)
     #pragma unroll
-    for (int t = 0; t < L::NB; t++) {
-        h8v vh[2];
-        f32x16 d = {};
+    for (int t = 0; t < L::NB; t += U) {
+        f32x16 d[U] = {};
+        h8v vh[U][2];
         #pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const h8v vl = *reinterpret_cast<const h8v*>(vp + 32 * t * L::VRS + 64 + 32 * s);
-            vh[s] = *reinterpret_cast<const h8v*>(vp + 32 * t * L::VRS + 32 * s);
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, bh[s], d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[s], bl[s], d, 0, 0, 0);
+        for (int s = 0; s < 2; s++)
+            #pragma unroll
+            for (int u = 0; u < U; u++) {
+                const h8v vl = *reinterpret_cast<const h8v*>(vp + 32 * (t + u) * L::VRS + 64 + 32 * s);
+                vh[u][s] = *reinterpret_cast<const h8v*>(vp + 32 * (t + u) * L::VRS + 32 * s);
+                d[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, bh[s], d[u], 0, 0, 0);
+                d[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[u][s], bl[s], d[u], 0, 0, 0);
+            }
+        #pragma unroll
+        for (int u = 0; u < U; u++) {
+            d[u] *= 0x1p-11f;
+            #pragma unroll
+            for (int s = 0; s < 2; s++) d[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[u][s], bh[s], d[u], 0, 0, 0);
         }
         #pragma unroll
-        for (int s = 0; s < 2; s++) d = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[s], bh[s], d, 0, 0, 0);
-        o[t] += d;
+        for (int u = 0; u < U; u++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++) o[t + u][r] = __builtin_fmaf(d[u][r], inv, o[t + u][r]);
     }
 }
 
@@ -596,6 +651,7 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
         const_cast<float*>(a.v + (size_t)hk * a.head_stride), (short)0, (int)((uint32_t)a.kv_len * (4u * HD)), 0x00020000);
     ApRegs<HD> reg;
     uint32_t ve = 0;
+    bool bad = false;
     ap_load<HD>(reg, kr, vr, b_lo, t);
 
     // the lane's query row: dims 16 s + 8 g .. + 7 of every step s
@@ -633,7 +689,7 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
     if (t < 2) reinterpret_cast<int*>(lds + L::GROW)[t] = -1;
     ap_vmax<HD>(lds, reg, 0, t);
     __syncthreads();
-    ap_convert<HD>(lds, reg, 0, t, ve);
+    ap_convert<HD>(lds, reg, 0, t, ve, bad);
     if (nb > 1) {
         ap_load<HD>(reg, kr, vr, b_lo + 1, t);
         ap_vmax<HD>(lds, reg, 1, t);
@@ -645,25 +701,31 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
         // every wave is done with the other stage
         __syncthreads();
         const int grown = reinterpret_cast<const int*>(lds + L::GROW)[n & 1];
-        if (n + 1 < nb) ap_convert<HD>(lds, reg, n + 1, t, ve);
+        if (n + 1 < nb) ap_convert<HD>(lds, reg, n + 1, t, ve, bad);
         if (n + 2 < nb) ap_load<HD>(reg, kr, vr, b_lo + n + 2, t);
         const int j0 = 32 * (b_lo + n);
         ap_rescale<HD>(lds, n, __builtin_amdgcn_readfirstlane(grown), g, o);
         if (j0 < row.vis_last) ap_compute<HD>(lds, n, j0, qh, ql, qf, c, g, row, m, lsum, o);
         if (n + 2 < nb) ap_vmax<HD>(lds, reg, n & 1, t);
     }
-    // sums that are not finite: the whole tile again in f32 (0 * x is 0 or NaN)
+    // values too far apart, sums that are not finite: the whole tile again in
+    // f32 (0 * x is 0 or NaN)
     float z = lsum * 0.0f;
     #pragma unroll
     for (int u = 0; u < HD / 32; u++)
         #pragma unroll
         for (int r = 0; r < 16; r++) z = __builtin_fmaf(o[u][r], 0.0f, z);
-    if (__syncthreads_or(row.ok && z != 0.0f)) {
+    if (__syncthreads_or(bad || (row.ok && z != 0.0f))) {
         ap_rows_f32<HD>(lds, lds0, a, grp, tile, piece, b_lo, b_hi);
         return;
     }
     if (!row.ok) return;
-    if (piece >= 0 && g == 0) ap_store_ml<HD>(a, row, piece, m - AP_P, lsum);   // the p are against m - AP_P
+    // the sum into [1, 2) and O with it, so that O times V's scale stays in
+    // f32's range wherever its results do (m can lag by 2^32)
+    const uint32_t le = lsum > 0.0f ? __builtin_bit_cast(uint32_t, lsum) >> 23 : 127u;
+    const float dn = __builtin_bit_cast(float, (254u - le) << 23);
+    lsum *= dn;
+    if (piece >= 0 && g == 0) ap_store_ml<HD>(a, row, piece, m + (float)((int)le - 127), lsum);
     #pragma unroll
     for (int u = 0; u < HD / 32; u++)
         #pragma unroll
@@ -671,8 +733,8 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
             const int d = 32 * u + 8 * q + 4 * g;
             const float4 f = *reinterpret_cast<const float4*>(lds + L::VS + 4 * d);
             ap_store4<HD>(a, row, piece, d,
-                          make_float4(o[u][4 * q] * f.x, o[u][4 * q + 1] * f.y, o[u][4 * q + 2] * f.z, o[u][4 * q + 3] * f.w),
-                          lsum);
+                          make_float4(o[u][4 * q] * dn * f.x, o[u][4 * q + 1] * dn * f.y, o[u][4 * q + 2] * dn * f.z,
+                                      o[u][4 * q + 3] * dn * f.w), lsum);
         }
 }
 

@@ -148,3 +148,78 @@ def test_the_rule_changes_no_result(be, prompt_be, n_head, n_kv, hd, q_len, star
     rows.close()
     assert np.array_equal(outs[0], outs[1]) or np.array_equal(outs[0], outs[2])
     close(outs[1], outs[2], v, n_head)
+
+
+# ---- weights and values far apart ------------------------------------------------
+
+def exact(q, k, v, n_head):
+    """In 64 bits; the queries are the last ones."""
+    n_kv, kv_len, hd = k.shape
+    q_len = q.shape[1]
+    out = np.empty((q_len, n_head, hd))
+    with np.errstate(over="ignore", invalid="ignore"):
+        for h in range(n_head):
+            j = h * n_kv // n_head
+            s = q[h].astype(np.float64) @ k[j].astype(np.float64).T / np.sqrt(hd)
+            s[np.arange(kv_len)[None, :] > kv_len - q_len + np.arange(q_len)[:, None]] = -np.inf
+            p = np.exp(s - s.max(1, keepdims=True))
+            out[:, h] = p @ v[j].astype(np.float64) / p.sum(1, keepdims=True)
+    return out
+
+
+def sink(r, n_head, n_kv, q_len, kv_len, hd, at, gap):
+    """Every query scores position `at` `gap` nats above the largest other one."""
+    a = np.zeros(hd)
+    a[0] = 1.0
+    q = r.standard_normal((n_head, q_len, hd)) * 0.1
+    q[:, :, 0] = np.sqrt(hd)
+    k = r.standard_normal((n_kv, kv_len, hd))
+    k[:, at] = 0.0
+    k[:, at, 0] = np.delete(k[:, :, 0], at, 1).max(1) + gap
+    return q.astype(F32), k.astype(F32), r.standard_normal((n_kv, kv_len, hd)).astype(F32)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("kv_len,gap,top", [
+    (1024, 12, 0.0), (1024, 16, 0.0), (4096, 20, 0.0), (4096, 20, 1.0), (200, 12, 1e-6), (33, 12, 0.0),
+])
+def test_small_weights_keep_their_bits(prompt_be, hd, kv_len, gap, top):
+    """One position takes all but e^-gap of the weight and its V is `top` times
+    as large as the others': with 0 the results are the small weights' own.
+    Bar, relative to each head's results: a score of s nats rounds to s 2^-24,
+    and so does its weight's exponent; 2^-22 s leaves room for the products'
+    own roundings (s: the gap and 5 nats of the others' scores)."""
+    n_head, n_kv, q_len = 8, 2, 32
+    r = np.random.default_rng(kv_len + gap)
+    q, k, v = sink(r, n_head, n_kv, q_len, kv_len, hd, 0, gap)
+    v[:, 0] *= F32(top)
+    out, ref = attend_f32(prompt_be, q, k, v, n_head), exact(q, k, v, n_head)
+    for h in range(n_head):
+        # the first query of 33 positions sees two of them: rows on their own
+        err = np.linalg.norm(out[:, h] - ref[:, h], axis=1) / np.linalg.norm(ref[:, h], axis=1)
+        assert np.max(err) <= (gap + 5) * 2.0 ** -22, (h, float(np.max(err)))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("big", [1e4, 1e8, 1e10, 1e30, 3e38])
+@pytest.mark.parametrize("where", ["masked", "weightless", "grown", "first"])
+def test_values_beside_a_large_one(prompt_be, hd, big, where):
+    """A large finite V that a row gives no weight costs the row nothing: at a
+    later position of its block, at an earlier position whose weight is 0, or
+    in blocks that it sees nothing of.  "first": at the position that takes all
+    the weight, where the result is as large.  Bar 2e-6 of the largest |V| that
+    the row gives weight to, per dim."""
+    n_head, n_kv, q_len, kv_len = 8, 2, 90, 90
+    r = np.random.default_rng(int(np.log10(big)))
+    at = {"masked": 45, "weightless": 3, "grown": 70, "first": 0}[where]
+    q, k, v = sink(r, n_head, n_kv, q_len, kv_len, hd, at, -400.0 if where == "weightless" else 30.0 if where == "first" else 0.0)
+    v[:, at, 5:9] = F32(big)
+    rows = np.arange(at) if where in ("masked", "grown") else np.arange(at + 1, q_len) if where == "weightless" else np.arange(q_len)
+    out, ref = attend_f32(prompt_be, q, k, v, n_head), exact(q, k, v, n_head)
+    seen = np.abs(v[:, :kv_len]).copy()
+    if where != "first":
+        seen[:, at] = 0.0
+    for h in range(n_head):
+        top = np.maximum.accumulate(seen[h * n_kv // n_head], axis=0)[rows]
+        err = np.abs(out[rows, h] - ref[rows, h])
+        assert np.all(err <= 2e-6 * top), (h, float(np.max(err / top)))
