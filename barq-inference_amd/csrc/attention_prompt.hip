@@ -21,23 +21,28 @@
 // exactly), and a product takes three f16 MFMAs (hi hi, hi lo, lo hi; lo lo is
 // at most 2^-22 of it, 2^-24.6 root mean square) with f32 sums, 5.3 times the
 // f32 rate.  Scales keep the split away from f16's limits:
-//   K: per position, the row's largest |k| into [2^13, 2^14); the inverse
+//   K: per position, the row's largest |k| into [2^14, 2^15); the inverse
 //      multiplies the scores
 //   Q: per query row, the same
 //   P: per query row and block, the largest p just below 2^15
 //   V: per output dim, the largest |v| so far into [2^14, 2^15); the scale
 //      only ever shrinks, and O's dim is multiplied by the ratio when it does
-// f16 steps end at 2^-24.  K's and Q's elements below 2^-14 of the largest
-// they share a scale with therefore lose bits.  Weights and values spread
-// further (a first position that takes nearly all the weight; a large value
-// that a row does not see), and what they lose is not small against the
-// result when the large ones add little to it.  lo of P and V is held times
-// 2^11, so that its steps end at 2^-35: weights down to 2^-26 of their block's
-// largest (18 nats) and values down to 2^-25 keep all bits.  Weights further
-// down lose one per halving (in that block alone); a tile with values below
-// 2^-34 of their dim's scale, or with a scale that shrinks by more than that,
-// is computed again by ap_rows_f32, on f32 MFMAs without scales, and so is one
-// whose sums are not finite (infinities and NaN turn into NaN here).
+// f16 steps end at 2^-24.  K's and Q's elements below 2^-15 of the largest
+// they share a scale with therefore lose bits: up to 2^-39 of the row's
+// largest each, and of their score in log2 units about 2^-41 |k||q| (root mean
+// square over 128 normal dims, |k| and |q| the rows' largest).  Below |k||q| =
+// 2^18 that is 2^-23, what f32 rounds a score of 4 to; a tile with larger ones
+// (or with |k| from 2^74 on, whose scores could overflow before |q| is taken
+// into account) is computed again by ap_rows_f32, on f32 MFMAs without scales.
+// Weights and values spread further (a first position that takes nearly all
+// the weight; a large value that a row does not see), and what they lose is
+// not small against the result when the large ones add little to it.  lo of P
+// and V is held times 2^11, so that its steps end at 2^-35: weights down to
+// 2^-26 of their block's largest (18 nats) and values down to 2^-25 keep all
+// bits.  Weights further down lose one per halving (in that block alone); a
+// tile with values below 2^-34 of their dim's scale, or with a scale that
+// shrinks by more than that, goes to ap_rows_f32 too, and so does one whose
+// sums are not finite (infinities and NaN turn into NaN here).
 //
 // Data movement: a block's K and V rows are loaded into registers one block
 // ahead of the conversion, converted by all four waves and stored as f16 in
@@ -162,11 +167,13 @@ struct ApLds {
     static constexpr int VMAX = 2 * STAGE;    // [2][PARTS][HD]
     static constexpr int VR = VMAX + 2 * PARTS * HD * 4;   // [2][HD]
     static constexpr int GROW = VR + 2 * HD * 4;           // [2]: the last block of that parity with a rescale
-    static constexpr int VS = GROW + 16;      // [HD]
+    static constexpr int QM = GROW + 16;      // [AP_NW]: the waves' largest |q|
+    static constexpr int VS = QM + 16;        // [HD]
     static constexpr int F32_RS = 4 * HD + 16, F32_PIECES = HD / 4 + 1, F32_BLK = 32 * F32_RS;
     static constexpr int TOTAL = VS + 4 * HD;
     static_assert(4 * F32_BLK <= TOTAL, "the f32 stages fit");
     static_assert(8 / AP_NW * TOTAL <= 163840, "eight waves per CU");
+    static_assert(AP_NW == 4, "four waves' largest |q|");
     static_assert(PP >= 4 && HD % (4 * TPR) == 0, "whole float4 loads and position groups");
 };
 
@@ -385,8 +392,9 @@ __device__ __forceinline__ float ap_scale(uint32_t e) { return __builtin_bit_cas
 template <int P>
 __device__ __forceinline__ float ap_unscale(uint32_t e) { return __builtin_bit_cast(float, (e - P) << 23); }
 
-constexpr int AP_KQ = 13, AP_V = 14;
+constexpr int AP_KQ = 14, AP_V = 14;
 constexpr int AP_P = 2;               // the largest p before its scale: its exponents are then near 0, where f32 is finest
+constexpr uint32_t AP_SCORE = 18;     // log2 of the |k||q| from which scores are left to the f32 kernel
 constexpr uint32_t AP_SPREAD = 34;    // octaves below a dim's largest |v| that the split takes
 
 template <int HD>
@@ -422,10 +430,11 @@ __device__ __forceinline__ void ap_vmax(uint8_t* lds, const ApRegs<HD>& r, int p
 }
 
 // The loaded block n as f16 hi and lo into its stage.  ve: the exponent state
-// of the thread's dim (0: nothing but zeros so far).  bad: set when the thread's
-// values spread further than the split can hold.
+// of the thread's dim (0: nothing but zeros so far).  ke_max: the largest
+// exponent of its K rows.  bad: set when its values spread further than the
+// split can hold.
 template <int HD>
-__device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, int n, int t, uint32_t& ve, bool& bad) {
+__device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, int n, int t, uint32_t& ve, uint32_t& ke_max, bool& bad) {
     using L = ApLds<HD>;
     uint8_t* st = lds + (n & 1) * L::STAGE;
     const float mo = ap_minus_one();
@@ -443,6 +452,7 @@ __device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, in
         #pragma unroll
         for (int j = 0; j < 4; j++) km = fmaxf(km, __builtin_fabsf(r.k[i][j]));
     const uint32_t ke = ap_exp(group_max<L::TPR>(km));
+    ke_max = ke > ke_max ? ke : ke_max;
     const float ks = ap_scale<AP_KQ>(ke);
     uint8_t* krow = st + (t / L::TPR) * L::KRS + 8 * (t % L::TPR);
     #pragma unroll
@@ -650,7 +660,7 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
     const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(a.v + (size_t)hk * a.head_stride), (short)0, (int)((uint32_t)a.kv_len * (4u * HD)), 0x00020000);
     ApRegs<HD> reg;
-    uint32_t ve = 0;
+    uint32_t ve = 0, ke_max = 0;
     bool bad = false;
     ap_load<HD>(reg, kr, vr, b_lo, t);
 
@@ -671,7 +681,10 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
             qm = fmaxf(fmaxf(fmaxf(qm, __builtin_fabsf(qv[s].x)), fmaxf(__builtin_fabsf(qv[s].y), __builtin_fabsf(qv[s].z))),
                        __builtin_fabsf(qv[s].w));
         auto hb = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, qm), __builtin_bit_cast(int, qm), false, false);
-        const uint32_t qe = ap_exp(fmaxf(__builtin_bit_cast(float, (int)hb[0]), __builtin_bit_cast(float, (int)hb[1])));
+        qm = fmaxf(__builtin_bit_cast(float, (int)hb[0]), __builtin_bit_cast(float, (int)hb[1]));
+        const uint32_t qe = ap_exp(qm);
+        qm = group_max<32>(qm);
+        if (l == 0) reinterpret_cast<float*>(lds + L::QM)[wave] = qm;
         const float qs = ap_scale<AP_KQ>(qe), mo = ap_minus_one();
         qf = ap_unscale<AP_KQ>(qe) * a.scale;
         #pragma unroll
@@ -689,7 +702,7 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
     if (t < 2) reinterpret_cast<int*>(lds + L::GROW)[t] = -1;
     ap_vmax<HD>(lds, reg, 0, t);
     __syncthreads();
-    ap_convert<HD>(lds, reg, 0, t, ve, bad);
+    ap_convert<HD>(lds, reg, 0, t, ve, ke_max, bad);
     if (nb > 1) {
         ap_load<HD>(reg, kr, vr, b_lo + 1, t);
         ap_vmax<HD>(lds, reg, 1, t);
@@ -701,7 +714,7 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
         // every wave is done with the other stage
         __syncthreads();
         const int grown = reinterpret_cast<const int*>(lds + L::GROW)[n & 1];
-        if (n + 1 < nb) ap_convert<HD>(lds, reg, n + 1, t, ve, bad);
+        if (n + 1 < nb) ap_convert<HD>(lds, reg, n + 1, t, ve, ke_max, bad);
         if (n + 2 < nb) ap_load<HD>(reg, kr, vr, b_lo + n + 2, t);
         const int j0 = 32 * (b_lo + n);
         ap_rescale<HD>(lds, n, __builtin_amdgcn_readfirstlane(grown), g, o);
@@ -710,6 +723,9 @@ __device__ __forceinline__ void ap_tile(uint8_t* lds, uint32_t lds0, const ApArg
     }
     // values too far apart, sums that are not finite: the whole tile again in
     // f32 (0 * x is 0 or NaN)
+    const float* qw = reinterpret_cast<const float*>(lds + L::QM);
+    const uint32_t qe = ap_exp(fmaxf(fmaxf(qw[0], qw[1]), fmaxf(qw[2], qw[3])));
+    bad |= ke_max + qe >= 2u * 127u + AP_SCORE || ke_max > 200u;
     float z = lsum * 0.0f;
     #pragma unroll
     for (int u = 0; u < HD / 32; u++)

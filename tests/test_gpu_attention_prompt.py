@@ -223,3 +223,28 @@ def test_values_beside_a_large_one(prompt_be, hd, big, where):
         top = np.maximum.accumulate(seen[h * n_kv // n_head], axis=0)[rows]
         err = np.abs(out[rows, h] - ref[rows, h])
         assert np.all(err <= 2e-6 * top), (h, float(np.max(err / top)))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("case", ["1e6", "1e8", "1e30", "huge keys", "huge queries"])
+def test_keys_and_queries_beside_large_elements(prompt_be, hd, case):
+    """A large key element that the queries do not touch (they are 0 there)
+    leaves the scores alone, and so do scales that only the product evens out.
+    Bar 4e-6 of the largest |V|: scores of 10 nats to 2^-22."""
+    n_head, n_kv, q_len, kv_len = 8, 2, 100, 160
+    r = np.random.default_rng(hd)
+    q, k, v = (r.standard_normal(s).astype(F32) for s in ((n_head, q_len, hd), (n_kv, kv_len, hd), (n_kv, kv_len, hd)))
+    if case == "huge keys":        # one row in ten, against tiny queries: ordinary scores
+        k[:, ::10] *= F32(1e33)
+        q *= F32(1e-33)
+    elif case == "huge queries":   # a query row in ten against keys that are all tiny
+        q[:, ::10] *= F32(1e33)
+        k *= F32(1e-33)
+    else:
+        q[:, :, 7] = 0.0
+        k[:, 20:120:3, 7] = F32(float(case))
+    out, ref = attend_f32(prompt_be, q, k, v, n_head), exact(q, k, v, n_head)
+    for h in range(n_head):
+        top = np.max(np.abs(v[h * n_kv // n_head]), axis=0)
+        err = np.abs(out[:, h] - ref[:, h])
+        assert np.all(err <= 4e-6 * top), (h, float(np.max(err / top)))
