@@ -316,12 +316,41 @@ __device__ __forceinline__ void ap_rows_f32(const uint8_t* lds, uint32_t lds0, c
         lsum = lsum * corr + rs;
         #pragma unroll
         for (int t = 0; t < NB; t++) o[t] *= corr;
+        bool inf_or_nan = false;
         #pragma unroll
         for (int st = 0; st < 16; st++) {
             const int kv = 8 * (st >> 2) + 4 * g + (st & 3);
             const fvec vv = *reinterpret_cast<const fvec*>(vs + kv * L::F32_RS + 4 * NB * c);
             #pragma unroll
-            for (int t = 0; t < NB; t++) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[t], p[st], o[t], 0, 0, 0);
+            for (int t = 0; t < NB; t++) {
+                const bool finite = __builtin_fabsf(vv[t]) < INFINITY;
+                inf_or_nan |= !finite;
+                o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(finite ? vv[t] : 0.0f, p[st], o[t], 0, 0, 0);
+            }
+        }
+        // Infinities and NaN in V only go to the rows that see their position
+        // (in a product 0 * inf would be NaN for the others).
+        if (__any(inf_or_nan)) {
+            #pragma unroll 1
+            for (int st = 0; st < 16; st++) {
+                float ps = p[0];
+                #pragma unroll
+                for (int u = 1; u < 16; u++) ps = st == u ? p[u] : ps;
+                const auto pp = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, ps), __builtin_bit_cast(int, ps), false, false);
+                #pragma unroll
+                for (int h = 0; h < 2; h++) {   // the positions of the two half-waves
+                    const int kv = 8 * (st >> 2) + 4 * h + (st & 3);
+                    const float ph = __builtin_bit_cast(float, (int)pp[h]);
+                    const bool seen = j0 + kv < row.vis;
+                    #pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const fvec vv = *reinterpret_cast<const fvec*>(vs + kv * L::F32_RS + 4 * NB * (8 * (r >> 2) + 4 * g + (r & 3)));
+                        #pragma unroll
+                        for (int t = 0; t < NB; t++)
+                            if (seen && !(__builtin_fabsf(vv[t]) < INFINITY)) o[t][r] = __builtin_fmaf(ph, vv[t], o[t][r]);
+                    }
+                }
+            }
         }
     }
     if (!row.ok) return;

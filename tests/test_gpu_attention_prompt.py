@@ -248,3 +248,28 @@ def test_keys_and_queries_beside_large_elements(prompt_be, hd, case):
         top = np.max(np.abs(v[h * n_kv // n_head]), axis=0)
         err = np.abs(out[:, h] - ref[:, h])
         assert np.all(err <= 4e-6 * top), (h, float(np.max(err / top)))
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("q_len,start,at", [(70, 0, 5), (70, 0, 40), (8, 300, 305), (100, 600, 640)])
+def test_infinities_and_nan_that_only_later_rows_see(prompt_be, orc, hd, q_len, start, at):
+    """Infinities and NaN in V and K at position `at` change no earlier row, also
+    of its block of 32 positions, and no other dim or head; the last case runs
+    in pieces."""
+    n_head, n_kv, kv_len = 8, 2, start + q_len
+    r = np.random.default_rng(q_len + at)
+    q, k, v = (r.standard_normal(s).astype(F32) for s in ((n_head, q_len, hd), (n_kv, kv_len, hd), (n_kv, kv_len, hd)))
+    ref = orc.attention(q, k, v, n_head, q_len, kv_len, start)
+    bad = v.copy()
+    bad[0, at, 9], bad[0, at, 10], bad[0, at, 11] = np.inf, -np.inf, np.nan
+    out = attend_f32(prompt_be, q, k, bad, n_head)
+    late = np.arange(q_len) >= at - start
+    assert np.all(np.isposinf(out[late, :4, 9])) and np.all(np.isneginf(out[late, :4, 10])) and np.all(np.isnan(out[late, :4, 11]))
+    out[late, :4, 9:12] = ref[late, :4, 9:12]
+    close(out, ref, v, n_head)
+    bad = k.copy()
+    bad[1, at, 3] = np.nan
+    out = attend_f32(prompt_be, q, bad, v, n_head)
+    assert np.all(np.isnan(out[late, 4:]))
+    out[late, 4:] = ref[late, 4:]
+    close(out, ref, v, n_head)
