@@ -57,16 +57,13 @@
 // one scale per row for P and no look at V's spread: 190 / 68 / 37 / 24 / 25.
 // P V on f32 MFMAs: 317 / 100 / 48 / 27 / 28.)  Error against 64 bits (relative
 // 2-norm, the same calls) 1.6e-7 to 1.9e-7 against 2.0e-7 to 3.9e-7.
+#include "attention_prompt_plan.hpp"
 #include "common.hpp"
 #include "launch.hpp"
 #include "mfma_common.hpp"
 #include "q8k_block.hpp"
 
 #include <cmath>
-#include <functional>
-#include <queue>
-#include <utility>
-#include <vector>
 
 namespace barq {
 
@@ -76,22 +73,12 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4n __attribute__((ext_vector_type(4)));
 
 constexpr float LOG2E = 1.44269504088896340736f;
-constexpr int AP_NW = 4, AP_ROWS = 32 * AP_NW;   // waves of a workgroup, query rows of its tile
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Position blocks of 32 that tile `tile` of a kv head's flattened rows sees.
-__host__ __device__ __forceinline__ int ap_tile_blocks(int tile, int G, int q_len, int kv_len, long long start_pos) {
-    const int row = tile * AP_ROWS + AP_ROWS - 1;
-    const int i_last = row / G < q_len - 1 ? row / G : q_len - 1;
-    const long long vis_last = start_pos + i_last + 1;
-    const int j_end = (int)(vis_last < kv_len ? vis_last : kv_len);
-    return (j_end + 31) / 32;
-}
-
-// The merge of a row's pieces: one wave per 256 output values (the 256 / HD
-// heads of one Q8_K block of row i), four values per lane; Q8 writes the
-// block's Q8_K bytes (q8_k_block) instead of the f32 values.  One pass over
+// The merge of a row's pieces: one wave per 256 output values (256 / HD heads
+// of row i; fewer in a last wave), four values per lane; Q8, whose rows are
+// whole blocks, writes the values' Q8_K block (q8_k_block) instead of them.  One pass over
 // the pieces, each rescaling what was summed before it, so a row waits for
 // memory once per two pieces and not twice per piece (2048 tokens in two
 // pieces per long tile: see attn_prompt_plan).
@@ -99,11 +86,12 @@ template <int HD, bool Q8>
 __global__ __launch_bounds__(256)
 void attn_combine_few_kernel(const float* __restrict__ part, int stride, int chunk, int n_head, int G, int q_len,
                              int kv_len, long long start_pos, float* __restrict__ out, uint8_t* __restrict__ out_q8) {
-    const int nblk = n_head * HD / 256;
+    const int nblk = (n_head * HD + 255) / 256;
     const int b = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = blockIdx.y;
     if (b >= nblk) return;
     const int l = threadIdx.x & 63;
     const int h = b * (256 / HD) + 4 * l / HD, d = 4 * l % HD;
+    if (!Q8 && h >= n_head) return;
     // the pieces of the row's tile (attn_prompt_kernel's list)
     const int tile = (i * G + h % G) / AP_ROWS;
     const int n_split = (ap_tile_blocks(tile, G, q_len, kv_len, start_pos) + chunk - 1) / chunk;
@@ -810,149 +798,8 @@ void attn_prompt_kernel(ApArgs a) {
 
 // ---- launch ------------------------------------------------------------------
 
-// Whether a chunk takes this kernel: head_dim 64 or 128, a kv head's rows
-// addressable by the 32-bit buffer offsets of its K/V loads, and enough work
-// for its longer fixed part.  The decode kernel (attention.hip) runs each
-// query row by itself: a row costs its products at 5.5 Tera multiply-adds/s
-// (QK and PV counted once) or its K and V rows from L2 at 14 TB/s (read once
-// per kv head for groups of 2, 4 or 8 query heads, else once per query head).
-// This kernel starts about 12 us later and reads K and V once, at 3.5 TB/s
-// with the conversion.  Measured, us per call, decode kernel / this one:
-// 32/8 heads of 128, 4000 cached, 6 / 8 / 12 rows 24.6 / 26.7, 30.0 / 27.2,
-// 42.1 / 28.3; 500 cached, 24 / 40 rows 14.0 / 19.6, 21.5 / 21.2; 32/32 heads,
-// 4000 cached, 4 / 6 rows 43.6 / 47.5, 69.5 / 47.4; 24/8 heads, 2 / 3 rows
-// 24.4 / 25.6, 31.8 / 25.9; 32/8 heads of 64, 8 / 12 rows 19.1 / 19.6, 24.9 /
-// 20.9; 40 rows from position 0: 7.7 / 15.8.  BARQ_ATTN_MFMA_MIN_Q: this
-// kernel from that many rows on, whatever the work.
 bool attn_prompt_path(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {
-    if ((head_dim != 64 && head_dim != 128) || kv_len >= ((size_t)1 << 23)) return false;
-    const int min_q = tuning_env(TUNE_ATTN_MFMA_MIN_Q);
-    if (min_q > 0) return q_len >= (size_t)min_q;
-    if (q_len < 2) return false;
-    const size_t g = n_head_kv && n_head % n_head_kv == 0 ? n_head / n_head_kv : 1;
-    const double reads = (double)(g == 2 || g == 4 || g == 8 ? n_head_kv : n_head);   // of K and V per query row
-    const double seen = (double)kv_len - (q_len < kv_len ? 0.5 * (double)q_len : 0.5 * (double)kv_len);
-    const double by_macs = (double)n_head / 5.5e6, by_bytes = reads * 8.0 / 14e6;   // us per position and dim
-    const double rows_us = (double)q_len * seen * (double)head_dim * (by_macs > by_bytes ? by_macs : by_bytes);
-    return rows_us > 1.2 * (12.0 + (double)kv_len * (double)(n_head_kv * head_dim) * 8.0 / 3.5e6);
-}
-
-// Launch plan: whole tiles, or pieces of `chunk` position blocks (partial
-// states merged by attn_combine_few_kernel).  The plan assumes the chunk's queries are the
-// last q_len of the kv_len positions (a prompt); at launch only the piece
-// counts follow the actual start position, within `stride` pieces per tile
-// (the workspace bound).
-struct ApPlan {
-    int G;        // query heads per kv head (1 when they do not divide)
-    int groups;
-    int tiles;    // per group
-    int chunk;    // position blocks per piece; 0: whole tiles, no partial states
-    int stride;   // partial states per (query row, head)
-};
-
-static ApPlan attn_prompt_plan_uncached(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {
-    ApPlan p{};
-    p.G = (int)(n_head_kv && n_head % n_head_kv == 0 ? n_head / n_head_kv : 1);
-    p.groups = (int)(n_head / p.G);
-    p.tiles = (int)((q_len * p.G + AP_ROWS - 1) / AP_ROWS);
-    const size_t cus = (size_t)cu_count_attn();
-    p.chunk = 0;
-    p.stride = 1;
-    // the merge writes whole Q8_K blocks (256 values); and where the tiles
-    // alone give every CU two workgroups, pieces only cost (2048 tokens,
-    // Llama-3-8B heads: 162 us whole, 200 us with the longer half cut in two)
-    if ((n_head * head_dim) % 256 != 0 || (size_t)p.tiles * p.groups >= 2 * cus) return p;
-    const long long start = kv_len > q_len ? (long long)(kv_len - q_len) : 0;
-    std::vector<int> nbs(p.tiles);
-    int longest = 0;
-    for (int t = 0; t < p.tiles; t++) {
-        nbs[t] = ap_tile_blocks(t, p.G, (int)q_len, (int)kv_len, start);
-        longest = nbs[t] > longest ? nbs[t] : longest;
-    }
-    // Choose the chunk by simulating the launch in units of one position block
-    // (about 2 us): the pieces in the kernel's order (each costing its blocks
-    // + FIXED for its fixed part: the query rows, the first loads, the partial
-    // state), every CU holding up to two workgroups that share it equally,
-    // each further piece going to the CU that frees a slot first; and the
-    // partial states' way to memory and back (MERGE units per byte, about 4
-    // TB/s).  Candidates cut the longest tile into k = 1, 2, ... pieces while
-    // there are at most four pieces per CU in all (more never measured
-    // faster); ties keep fewer pieces.
-    constexpr double FIXED = 1.5, MERGE = 2.0 / 4e6 / 2.0;
-    const double part_bytes = (double)AP_ROWS * p.groups * (head_dim + 2) * sizeof(float);
-    auto simulate = [&](int c) {
-        struct Cu { double t, w[2]; int n; };
-        std::vector<Cu> cu(cus, Cu{0.0, {0.0, 0.0}, 0});
-        auto event = [](const Cu& u) {
-            return u.n == 2 ? u.t + 1.7 * (u.w[0] < u.w[1] ? u.w[0] : u.w[1]) : u.t + u.w[0];
-        };
-        typedef std::pair<double, size_t> Ev;
-        std::priority_queue<Ev, std::vector<Ev>, std::greater<Ev>> heap;
-        double end = 0.0, merged = 0.0;
-        size_t placed = 0;
-        auto finish = [&]() {   // the next piece to end; its CU has a slot free
-            const Ev ev = heap.top();
-            heap.pop();
-            Cu& u = cu[ev.second];
-            if (u.n == 2) {   // the shorter piece ends; the other has done as much
-                const int done = u.w[0] < u.w[1] ? 0 : 1;
-                u.w[0] = u.w[1 - done] - u.w[done];
-                u.n = 1;
-            } else {
-                u.n = 0;
-            }
-            u.t = ev.first;
-            end = ev.first > end ? ev.first : end;
-            return ev.second;
-        };
-        for (int t = p.tiles - 1; t >= 0; t--) {   // the kernel's order: longest tiles first, then the head groups
-            if (nbs[t] > c) merged += (nbs[t] + c - 1) / c * part_bytes;
-            for (int b = 0; b < nbs[t]; b += c)
-                for (int g = 0; g < p.groups; g++) {
-                    const double len = (nbs[t] - b < c ? nbs[t] - b : c) + FIXED;
-                    if (placed < 2 * cus) {   // the first round: one per CU, then a second
-                        Cu& u = cu[placed % cus];
-                        u.w[u.n++] = len;
-                        if (++placed == 2 * cus)
-                            for (size_t k = 0; k < cus; k++) heap.push(Ev(event(cu[k]), k));
-                        continue;
-                    }
-                    const size_t k = finish();
-                    cu[k].w[cu[k].n++] = len;
-                    heap.push(Ev(event(cu[k]), k));
-                }
-        }
-        if (placed < 2 * cus)
-            for (size_t k = 0; k < cus; k++)
-                if (cu[k].n) heap.push(Ev(event(cu[k]), k));
-        while (!heap.empty()) {
-            const size_t k = finish();
-            if (cu[k].n) heap.push(Ev(event(cu[k]), k));
-        }
-        return end + MERGE * merged;
-    };
-    size_t chunk = (size_t)longest;
-    const int ovr = tuning_env(TUNE_ATTN_MFMA_SPLIT);   // pieces of the longest tile (tuning)
-    double best = ovr > 0 ? 0.0 : simulate(longest);
-    for (int k = 2; ovr <= 0 && k <= longest; k++) {
-        const int c = (longest + k - 1) / k;
-        if ((size_t)c >= chunk) continue;
-        size_t n = 0;
-        for (int nb : nbs) n += (size_t)((nb + c - 1) / c);
-        if (n * p.groups > 4 * cus) break;   // smaller chunks only add pieces
-        const double e = simulate(c);
-        if (e < best - 1e-9) {
-            best = e;
-            chunk = (size_t)c;
-        }
-    }
-    if (ovr > 0) chunk = ((size_t)longest + (size_t)ovr - 1) / (size_t)ovr;
-    if (chunk < 1) chunk = 1;
-    if (chunk >= (size_t)longest) return p;   // every tile in one piece
-    const size_t nbmax = (kv_len + 31) / 32;
-    p.chunk = (int)chunk;
-    p.stride = (int)((nbmax + chunk - 1) / chunk);
-    return p;
+    return ap_path(n_head, n_head_kv, head_dim, q_len, kv_len, tuning_env(TUNE_ATTN_MFMA_MIN_Q));
 }
 
 // The plan of the last shape and device this thread asked for: the workspace
@@ -965,13 +812,14 @@ static ApPlan attn_prompt_plan(size_t n_head, size_t n_head_kv, size_t head_dim,
         bool valid;
     };
     thread_local Entry last = {{0, 0, 0, 0, 0}, -1, ApPlan{}, false};
-    if (tuning_env(TUNE_ATTN_MFMA_SPLIT) > 0) return attn_prompt_plan_uncached(n_head, n_head_kv, head_dim, q_len, kv_len);
+    const int ovr = tuning_env(TUNE_ATTN_MFMA_SPLIT);   // pieces of the longest tile (tuning)
+    if (ovr > 0) return ap_plan(n_head, n_head_kv, head_dim, q_len, kv_len, (size_t)cu_count_attn(), ovr);
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) dev = -1;
     if (last.valid && last.dev == dev && last.key[0] == n_head && last.key[1] == n_head_kv && last.key[2] == head_dim &&
         last.key[3] == q_len && last.key[4] == kv_len)
         return last.plan;
-    const ApPlan p = attn_prompt_plan_uncached(n_head, n_head_kv, head_dim, q_len, kv_len);
+    const ApPlan p = ap_plan(n_head, n_head_kv, head_dim, q_len, kv_len, (size_t)cu_count_attn(), 0);
     last = Entry{{n_head, n_head_kv, head_dim, q_len, kv_len}, dev, p, true};
     return p;
 }
@@ -1015,8 +863,7 @@ static hipError_t attn_prompt_launch_t(const AttnArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(attn_prompt_kernel<HD>, dim3(n * (unsigned)p.groups), dim3(64 * AP_NW), 0, s, k);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.chunk == 0) return e;
-    // (the plan splits only when the rows are whole Q8_K blocks)
-    const dim3 cg((unsigned)((a.n_head * HD / 256 + 3) / 4), (unsigned)a.q_len);
+    const dim3 cg((unsigned)(((a.n_head * HD + 255) / 256 + 3) / 4), (unsigned)a.q_len);
     if (a.out_q8)
         hipLaunchKernelGGL((attn_combine_few_kernel<HD, true>), cg, dim3(256), 0, s, a.part, p.stride, p.chunk,
                            (int)a.n_head, p.G, (int)a.q_len, (int)a.kv_len, (long long)a.start_pos, a.out, a.out_q8);

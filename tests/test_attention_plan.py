@@ -1,0 +1,75 @@
+"""The host side of prompt attention (csrc/attention_prompt_plan.hpp), compiled
+on its own: how the calls that its rule takes are cut into workgroups."""
+import os
+import random
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "barq-inference_amd", "csrc")
+CUS = 256
+
+MAIN = r"""
+#include "attention_prompt_plan.hpp"
+#include <algorithm>
+#include <cstdio>
+using namespace barq;
+// shapes on stdin -> taken, G, groups, tiles, chunk, stride, blocks of every tile
+int main() {
+    long long nh, nkv, hd, q, kv;
+    while (scanf("%lld %lld %lld %lld %lld", &nh, &nkv, &hd, &q, &kv) == 5) {
+        const ApPlan p = ap_plan(nh, nkv, hd, q, kv, 256, 0);
+        printf("%d %d %d %d %d %d", (int)ap_path(nh, nkv, hd, q, kv, 0), p.G, p.groups, p.tiles, p.chunk, p.stride);
+        for (int t = 0; t < p.tiles; t++) printf(" %d", ap_tile_blocks(t, p.G, q, kv, kv > q ? kv - q : 0));
+        printf("\n");
+    }
+}
+"""
+
+HEADS = [(32, 8), (32, 4), (32, 32), (24, 8), (16, 8), (8, 1), (14, 2), (71, 1), (15, 5), (6, 4), (9, 3), (1, 1), (3, 1)]
+
+
+def shapes():
+    r = random.Random(3)
+    out = [(14, 2, 64, 8, 4000), (71, 1, 64, 4, 4000), (15, 5, 64, 16, 4000), (32, 8, 128, 8, 4000), (8, 1, 128, 64, 131072),
+           (32, 8, 128, 2048, 2048), (32, 8, 64, 200, 1000), (1, 1, 64, 2, 100000)]
+    for _ in range(400):
+        q = int(round(2 ** r.uniform(1, 11)))
+        out.append((*r.choice(HEADS), r.choice([64, 128]), q, q + r.choice([0, int(round(2 ** r.uniform(4, 14)))])))
+    return out
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    src, exe = d / "main.cpp", d / "plan"
+    src.write_text(MAIN)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-I", CSRC, str(src), "-o", str(exe)], check=True)
+    text = "".join(" ".join(map(str, s)) + "\n" for s in shapes())
+    lines = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
+    rows = [list(map(int, line.split())) for line in lines]
+    return [(s, bool(r[0]), *r[1:6], r[6:]) for s, r in zip(shapes(), rows)]
+
+
+def test_tiles_cover_the_rows(plans):
+    for s, _, g, groups, tiles, chunk, stride, nbs in plans:
+        nh, nkv, _, q, kv = s
+        assert g * groups == nh and (nkv == groups or nh % nkv), s
+        assert len(nbs) == tiles and (tiles - 1) * 128 < q * g <= tiles * 128, s
+        assert max(nbs) == (kv + 31) // 32, s
+        # the workspace holds every piece, wherever the rows start
+        assert chunk == 0 and stride == 1 or chunk * stride >= (kv + 31) // 32 > chunk, s
+
+
+def test_calls_that_the_rule_takes_fill_the_cus(plans):
+    """No workgroup walks much more than a CU's share of the position blocks: at
+    most twice that (two workgroups share a CU) and three blocks of fixed part."""
+    taken = 0
+    for s, take, _, groups, _, chunk, _, nbs in plans:
+        if not take:
+            continue
+        taken += 1
+        share = sum(nbs) * groups / CUS
+        assert max(nbs) <= 2 * share + 3 or (0 < chunk <= 2 * share + 3), (s, chunk, max(nbs), share)
+    assert taken > 100

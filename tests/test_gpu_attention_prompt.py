@@ -273,3 +273,20 @@ def test_infinities_and_nan_that_only_later_rows_see(prompt_be, orc, hd, q_len, 
     assert np.all(np.isnan(out[late, 4:]))
     out[late, 4:] = ref[late, 4:]
     close(out, ref, v, n_head)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("n_head,n_kv,q_len,start", [(14, 2, 8, 700), (15, 5, 40, 300), (71, 1, 5, 400), (3, 1, 70, 200), (1, 1, 33, 100)])
+@pytest.mark.parametrize("pieces", [0, 3])
+def test_heads_of_no_whole_q8_k_blocks(orc, monkeypatch, hd, n_head, n_kv, q_len, start, pieces):
+    """Heads times dims that are no multiple of 256 in pieces too: the last wave
+    of the merge has rows of fewer heads."""
+    if pieces:
+        monkeypatch.setenv("BARQ_ATTN_MFMA_SPLIT", str(pieces))
+    b = backend(1)
+    r = np.random.default_rng(n_head)
+    kv_len = start + q_len
+    q, k, v = (r.standard_normal(s).astype(F32) for s in ((n_head, q_len, hd), (n_kv, kv_len, hd), (n_kv, kv_len, hd)))
+    out = attend_f32(b, q, k, v, n_head)
+    b.close()
+    close(out, orc.attention(q, k, v, n_head, q_len, kv_len, start), v, n_head)
