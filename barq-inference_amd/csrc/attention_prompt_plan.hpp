@@ -3,9 +3,6 @@
 #pragma once
 #include <stddef.h>
 
-#include <functional>
-#include <queue>
-#include <utility>
 #include <vector>
 
 #if defined(__HIPCC__)
@@ -67,6 +64,50 @@ struct ApPlan {
     int stride;   // partial states per (query row, head)
 };
 
+// A launch's time, us, if the tiles (runs of equal length, shortest first) are
+// cut into pieces of c position blocks: the last to end of the workgroups,
+// which take pieces in the list's order, longest tile first, two to a CU, and
+// the merge.  A block takes 2.7 us with 128 dims and 1.35 with 64, a piece as
+// long as 1.4 blocks more for its fixed part (the query rows, the first loads,
+// the partial state), and two pieces that share a CU 1.2 times as long as one;
+// the merge reads a row's pieces one after the other (0.085 us each) and all
+// states go to memory and back at 2.3 TB/s.  Fitted on MI355X to 108 launches
+// of 14 shapes (2 to 1024 rows, 0 to 16000 cached, 1 to 32 kv heads): 11 % off
+// root mean square, and its choice is the fastest chunk measured for each.
+struct ApRun {
+    int blocks, tiles;
+    // pieces of c blocks, by 1 / c (an integer division takes several times as
+    // long, and a plan forms some thousand quotients; blocks < 2^18)
+    size_t pieces(double inv) const { return (size_t)(((double)blocks - 0.5) * inv + 1.0) * (size_t)tiles; }
+};
+inline double ap_time(const std::vector<ApRun>& runs, size_t groups, size_t head_dim, size_t cus, int c) {
+    constexpr double FIXED = 1.4, SHARE = 1.2, MERGE_PIECE = 0.085, MERGE_BYTE = 2.0 / 4.6e6;
+    const double block = head_dim == 128 ? 2.7 : 1.35;
+    const double inv = 1.0 / (double)c;
+    const auto length = [&](const ApRun& r) { return (double)(r.blocks < c ? r.blocks : c) + FIXED; };
+    size_t n = 0, merged = 0, blocks = 0;
+    for (const ApRun& r : runs) {
+        const size_t k = r.pieces(inv);
+        n += k;
+        if (r.blocks > c) merged += k;
+        blocks += (size_t)r.blocks * (size_t)r.tiles;
+    }
+    double t = length(runs.back());
+    if (n * groups > cus) {   // the longest piece shares its CU with the one cus places down the list
+        size_t left = cus / groups, i = runs.size() - 1;
+        while (i > 0 && runs[i].pieces(inv) <= left) left -= runs[i--].pieces(inv);
+        t += (SHARE - 1.0) * length(runs[i]);
+        double all = ((double)blocks + FIXED * (double)n) * (double)groups * SHARE / 2.0 / (double)cus;
+        if (n * groups > 2 * cus) all += 0.5 * SHARE * length(runs.front());   // the CUs end about half a last piece apart
+        t = t > all ? t : all;
+    }
+    t *= block;
+    if (merged)
+        t += MERGE_PIECE * (double)((runs.back().blocks + c - 1) / c) +
+             MERGE_BYTE * (double)(merged * AP_ROWS * groups * (head_dim + 2) * sizeof(float));
+    return t;
+}
+
 // pieces > 0: that many of the longest tile (tuning).
 inline ApPlan ap_plan(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len, size_t cus, int pieces) {
     ApPlan p{};
@@ -79,94 +120,52 @@ inline ApPlan ap_plan(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q
     // tokens, Llama-3-8B heads: 162 us whole, 200 us with the longer half cut in two)
     if ((size_t)p.tiles * p.groups >= 2 * cus) return p;
     const long long start = kv_len > q_len ? (long long)(kv_len - q_len) : 0;
-    std::vector<int> nbs(p.tiles);
-    int longest = 0;
+    std::vector<ApRun> runs;
+    runs.reserve((size_t)p.tiles);
+    size_t total = 0;
     for (int t = 0; t < p.tiles; t++) {
-        nbs[t] = ap_tile_blocks(t, p.G, (int)q_len, (int)kv_len, start);
-        longest = nbs[t] > longest ? nbs[t] : longest;
+        const int nb = ap_tile_blocks(t, p.G, (int)q_len, (int)kv_len, start);
+        if (!runs.empty() && runs.back().blocks == nb) runs.back().tiles++;
+        else runs.push_back(ApRun{nb, 1});
+        total += (size_t)nb;
     }
-    // Choose the chunk by simulating the launch in units of one position block
-    // (about 2 us): the pieces in the kernel's order (each costing its blocks
-    // + FIXED for its fixed part: the query rows, the first loads, the partial
-    // state), every CU holding up to two workgroups that share it equally,
-    // each further piece going to the CU that frees a slot first; and the
-    // partial states' way to memory and back (MERGE units per byte, about 4
-    // TB/s).  Candidates cut the longest tile into k = 1, 2, ... pieces while
-    // there are at most four pieces per CU in all (more never measured
-    // faster); ties keep fewer pieces.
-    constexpr double FIXED = 1.5, MERGE = 2.0 / 4e6 / 2.0;
-    const double part_bytes = (double)AP_ROWS * p.groups * (head_dim + 2) * sizeof(float);
-    auto simulate = [&](int c) {
-        struct Cu { double t, w[2]; int n; };
-        std::vector<Cu> cu(cus, Cu{0.0, {0.0, 0.0}, 0});
-        auto event = [](const Cu& u) {
-            return u.n == 2 ? u.t + 1.7 * (u.w[0] < u.w[1] ? u.w[0] : u.w[1]) : u.t + u.w[0];
-        };
-        typedef std::pair<double, size_t> Ev;
-        std::priority_queue<Ev, std::vector<Ev>, std::greater<Ev>> heap;
-        double end = 0.0, merged = 0.0;
-        size_t placed = 0;
-        auto finish = [&]() {   // the next piece to end; its CU has a slot free
-            const Ev ev = heap.top();
-            heap.pop();
-            Cu& u = cu[ev.second];
-            if (u.n == 2) {   // the shorter piece ends; the other has done as much
-                const int done = u.w[0] < u.w[1] ? 0 : 1;
-                u.w[0] = u.w[1 - done] - u.w[done];
-                u.n = 1;
-            } else {
-                u.n = 0;
+    const int longest = runs.back().blocks;
+    int chunk = longest;
+    if (pieces > 0) {
+        chunk = (longest + pieces - 1) / pieces;
+    } else {
+        // Candidates: the smallest chunks that leave at most 1/4, 1/2, ... 2, 2
+        // 1/2, ... 4 pieces per CU (more never measured faster).  Smaller chunks of as many
+        // rounds of pieces only add pieces to merge, larger ones make the pieces
+        // longer.  Ties keep the larger chunk.
+        double best = ap_time(runs, (size_t)p.groups, head_dim, cus, longest);
+        for (int k = 1; k <= 16; k += k < 8 ? 1 : 2) {
+            const size_t most = cus * (size_t)k / 4 / (size_t)p.groups;   // per head group
+            if (most <= (size_t)p.tiles) continue;
+            // n(c) = sum of ceil(blocks / c) lies between total / c and that + tiles
+            int lo = (int)((total + most - 1) / most), hi = (int)(total / (most - (size_t)p.tiles)) + 1;
+            if (lo < 1) lo = 1;
+            if (hi > longest) hi = longest;
+            while (lo < hi) {
+                const int mid = (lo + hi) / 2;
+                size_t n = 0;
+                for (const ApRun& r : runs) n += r.pieces(1.0 / (double)mid);
+                if (n <= most) hi = mid;
+                else lo = mid + 1;
             }
-            u.t = ev.first;
-            end = ev.first > end ? ev.first : end;
-            return ev.second;
-        };
-        for (int t = p.tiles - 1; t >= 0; t--) {   // the kernel's order: longest tiles first, then the head groups
-            if (nbs[t] > c) merged += (nbs[t] + c - 1) / c * part_bytes;
-            for (int b = 0; b < nbs[t]; b += c)
-                for (int g = 0; g < p.groups; g++) {
-                    const double len = (nbs[t] - b < c ? nbs[t] - b : c) + FIXED;
-                    if (placed < 2 * cus) {   // the first round: one per CU, then a second
-                        Cu& u = cu[placed % cus];
-                        u.w[u.n++] = len;
-                        if (++placed == 2 * cus)
-                            for (size_t k = 0; k < cus; k++) heap.push(Ev(event(cu[k]), k));
-                        continue;
-                    }
-                    const size_t k = finish();
-                    cu[k].w[cu[k].n++] = len;
-                    heap.push(Ev(event(cu[k]), k));
-                }
-        }
-        if (placed < 2 * cus)
-            for (size_t k = 0; k < cus; k++)
-                if (cu[k].n) heap.push(Ev(event(cu[k]), k));
-        while (!heap.empty()) {
-            const size_t k = finish();
-            if (cu[k].n) heap.push(Ev(event(cu[k]), k));
-        }
-        return end + MERGE * merged;
-    };
-    size_t chunk = (size_t)longest;
-    double best = pieces > 0 ? 0.0 : simulate(longest);
-    for (int k = 2; pieces <= 0 && k <= longest; k++) {
-        const int c = (longest + k - 1) / k;
-        if ((size_t)c >= chunk) continue;
-        size_t n = 0;
-        for (int nb : nbs) n += (size_t)((nb + c - 1) / c);
-        if (n * p.groups > 4 * cus) break;   // smaller chunks only add pieces
-        const double e = simulate(c);
-        if (e < best - 1e-9) {
-            best = e;
-            chunk = (size_t)c;
+            if (lo >= chunk) continue;
+            const double e = ap_time(runs, (size_t)p.groups, head_dim, cus, lo);
+            if (e < best - 1e-9) {
+                best = e;
+                chunk = lo;
+            }
         }
     }
-    if (pieces > 0) chunk = ((size_t)longest + (size_t)pieces - 1) / (size_t)pieces;
     if (chunk < 1) chunk = 1;
-    if (chunk >= (size_t)longest) return p;   // every tile in one piece
-    const size_t nbmax = (kv_len + 31) / 32;
-    p.chunk = (int)chunk;
-    p.stride = (int)((nbmax + chunk - 1) / chunk);
+    if (chunk >= longest) return p;   // every tile in one piece
+    const int nbmax = (int)((kv_len + 31) / 32);
+    p.chunk = chunk;
+    p.stride = (nbmax + chunk - 1) / chunk;
     return p;
 }
 

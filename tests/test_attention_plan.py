@@ -13,14 +13,21 @@ CUS = 256
 MAIN = r"""
 #include "attention_prompt_plan.hpp"
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 using namespace barq;
-// shapes on stdin -> taken, G, groups, tiles, chunk, stride, blocks of every tile
+// shapes on stdin -> taken, ns of a plan (best of five), G, groups, tiles, chunk, stride, blocks of every tile
 int main() {
     long long nh, nkv, hd, q, kv;
     while (scanf("%lld %lld %lld %lld %lld", &nh, &nkv, &hd, &q, &kv) == 5) {
-        const ApPlan p = ap_plan(nh, nkv, hd, q, kv, 256, 0);
-        printf("%d %d %d %d %d %d", (int)ap_path(nh, nkv, hd, q, kv, 0), p.G, p.groups, p.tiles, p.chunk, p.stride);
+        ApPlan p;
+        long long ns = 1LL << 60;
+        for (int i = 0; i < 5; i++) {
+            const auto t0 = std::chrono::steady_clock::now();
+            p = ap_plan(nh, nkv, hd, q, kv, 256, 0);
+            ns = std::min(ns, (long long)std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now() - t0).count());
+        }
+        printf("%d %lld %d %d %d %d %d", (int)ap_path(nh, nkv, hd, q, kv, 0), ns, p.G, p.groups, p.tiles, p.chunk, p.stride);
         for (int t = 0; t < p.tiles; t++) printf(" %d", ap_tile_blocks(t, p.G, q, kv, kv > q ? kv - q : 0));
         printf("\n");
     }
@@ -49,11 +56,11 @@ def plans(tmp_path_factory):
     text = "".join(" ".join(map(str, s)) + "\n" for s in shapes())
     lines = subprocess.run([str(exe)], input=text, capture_output=True, text=True, check=True).stdout.splitlines()
     rows = [list(map(int, line.split())) for line in lines]
-    return [(s, bool(r[0]), *r[1:6], r[6:]) for s, r in zip(shapes(), rows)]
+    return [(s, bool(r[0]), *r[1:7], r[7:]) for s, r in zip(shapes(), rows)]
 
 
 def test_tiles_cover_the_rows(plans):
-    for s, _, g, groups, tiles, chunk, stride, nbs in plans:
+    for s, _, _, g, groups, tiles, chunk, stride, nbs in plans:
         nh, nkv, _, q, kv = s
         assert g * groups == nh and (nkv == groups or nh % nkv), s
         assert len(nbs) == tiles and (tiles - 1) * 128 < q * g <= tiles * 128, s
@@ -66,10 +73,21 @@ def test_calls_that_the_rule_takes_fill_the_cus(plans):
     """No workgroup walks much more than a CU's share of the position blocks: at
     most twice that (two workgroups share a CU) and three blocks of fixed part."""
     taken = 0
-    for s, take, _, groups, _, chunk, _, nbs in plans:
+    for s, take, _, _, groups, _, chunk, _, nbs in plans:
         if not take:
             continue
         taken += 1
         share = sum(nbs) * groups / CUS
         assert max(nbs) <= 2 * share + 3 or (0 < chunk <= 2 * share + 3), (s, chunk, max(nbs), share)
     assert taken > 100
+
+
+def test_a_plan_takes_microseconds(plans):
+    """A server's shapes change with every step, so a plan is part of the call:
+    at most some 8 us on an idle core, half a microsecond for a few rows (a
+    simulation of the launch took 0.4 to 8 ms).  Bars four times that and more,
+    for a busy machine."""
+    for s, _, ns, *_ in plans:
+        assert ns < 40000, (s, ns)
+    few = [ns for s, _, ns, *_ in plans if s[3] <= 16]
+    assert sorted(few)[len(few) // 2] < 5000, sorted(few)
