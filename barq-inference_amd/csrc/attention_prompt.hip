@@ -592,21 +592,22 @@ __device__ __forceinline__ void ap_compute(const uint8_t* lds, int n, int j0, co
         auto hb = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, bm), __builtin_bit_cast(int, bm), false, false);
         bm = fmaxf(__builtin_bit_cast(float, (int)hb[0]), __builtin_bit_cast(float, (int)hb[1])) * qf;
     }
-    // The block's reference is bi (its p at most 2^AP_P, the largest above half of
-    // that); o and lsum are relative to m.  Both are whole numbers, so their
-    // factors are exact powers of two; m follows the maximum when that has grown
-    // by 2^32.
-    const float bi = __builtin_ceilf(bm);
-    if (__any(bi > m + 32.0f)) {
-        const float mn = fmaxf(m, bi);
+    // o and lsum are relative to m, the largest score when m was last moved, up to
+    // a multiple of 2^-14; it moves when the maximum has grown by 2^32.  A
+    // block's p are relative to m plus a whole number (exact, and so is the
+    // factor between the two), at most 2^AP_P.  A row's largest weight is then
+    // 2^AP_P itself while m is its score.
+    if (__any(bm > m + 32.0f)) {
+        const float mn = fmaxf(m, __builtin_ceilf(bm * 0x1p14f) * 0x1p-14f);
         const float corr = m == -INFINITY ? 0.0f : fast_exp2(m - mn);
         m = mn;
         lsum *= corr;
         #pragma unroll
         for (int t = 0; t < L::NB; t++) o[t] *= corr;
     }
-    const bool none = bi == -INFINITY;   // a row that sees no position of the block
-    const float pref = none ? 0.0f : bi - (float)AP_P, step = none ? 0.0f : fast_exp2(bi - (float)AP_P - m);
+    const bool none = bm == -INFINITY;   // a row that sees no position of the block
+    const float k = none ? 0.0f : __builtin_ceilf(bm - m) - (float)AP_P;
+    const float pref = none ? 0.0f : m + k, step = none ? 0.0f : fast_exp2(k);
     const float inv = step * (1.0f / (float)(1 << (15 - AP_P)));
     const ApExt ex = ap_ext();
     float rs[8];
