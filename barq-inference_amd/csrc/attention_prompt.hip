@@ -799,12 +799,8 @@ void attn_prompt_kernel(ApArgs a) {
 
 // ---- launch ------------------------------------------------------------------
 
-bool attn_prompt_path(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {
-    return ap_path(n_head, n_head_kv, head_dim, q_len, kv_len, tuning_env(TUNE_ATTN_MFMA_MIN_Q));
-}
-
-// The plan of the last shape and device this thread asked for: the workspace
-// query and the launch ask in turn.
+// The plan of the last shape and device this thread asked for: the choice of
+// the kernel, the workspace query and the launch ask in turn.
 static ApPlan attn_prompt_plan(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {
     struct Entry {
         size_t key[5];
@@ -823,6 +819,13 @@ static ApPlan attn_prompt_plan(size_t n_head, size_t n_head_kv, size_t head_dim,
     const ApPlan p = ap_plan(n_head, n_head_kv, head_dim, q_len, kv_len, (size_t)cu_count_attn(), 0);
     last = Entry{{n_head, n_head_kv, head_dim, q_len, kv_len}, dev, p, true};
     return p;
+}
+
+bool attn_prompt_path(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {
+    const int min_q = tuning_env(TUNE_ATTN_MFMA_MIN_Q);
+    if (!ap_supported(head_dim, kv_len) || q_len < (min_q > 0 ? (size_t)min_q : 2)) return false;
+    if (min_q > 0) return true;
+    return ap_path(n_head, n_head_kv, head_dim, q_len, kv_len, attn_prompt_plan(n_head, n_head_kv, head_dim, q_len, kv_len));
 }
 
 size_t attn_prompt_workspace(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {

@@ -25,32 +25,6 @@ BARQ_HOST_DEVICE int ap_tile_blocks(int tile, int G, int q_len, int kv_len, long
     return (j_end + 31) / 32;
 }
 
-// Whether a chunk takes this kernel: head_dim 64 or 128, a kv head's rows
-// addressable by the 32-bit buffer offsets of its K/V loads, and enough work
-// for its longer fixed part.  The decode kernel (attention.hip) runs each
-// query row by itself: a row costs its products at 5.5 Tera multiply-adds/s
-// (QK and PV counted once) or its K and V rows from L2 at 14 TB/s (read once
-// per kv head for groups of 2, 4 or 8 query heads, else once per query head).
-// This kernel starts about 12 us later and reads K and V once, at 3.5 TB/s
-// with the conversion.  Measured, us per call, decode kernel / this one:
-// 32/8 heads of 128, 4000 cached, 6 / 8 / 12 rows 24.6 / 26.7, 30.0 / 27.2,
-// 42.1 / 28.3; 500 cached, 24 / 40 rows 14.0 / 19.6, 21.5 / 21.2; 32/32 heads,
-// 4000 cached, 4 / 6 rows 43.6 / 47.5, 69.5 / 47.4; 24/8 heads, 2 / 3 rows
-// 24.4 / 25.6, 31.8 / 25.9; 32/8 heads of 64, 8 / 12 rows 19.1 / 19.6, 24.9 /
-// 20.9; 40 rows from position 0: 7.7 / 15.8.  BARQ_ATTN_MFMA_MIN_Q: this
-// kernel from that many rows on, whatever the work.
-inline bool ap_path(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len, int min_q) {
-    if ((head_dim != 64 && head_dim != 128) || kv_len >= ((size_t)1 << 23)) return false;
-    if (min_q > 0) return q_len >= (size_t)min_q;
-    if (q_len < 2) return false;
-    const size_t g = n_head_kv && n_head % n_head_kv == 0 ? n_head / n_head_kv : 1;
-    const double reads = (double)(g == 2 || g == 4 || g == 8 ? n_head_kv : n_head);   // of K and V per query row
-    const double seen = (double)kv_len - (q_len < kv_len ? 0.5 * (double)q_len : 0.5 * (double)kv_len);
-    const double by_macs = (double)n_head / 5.5e6, by_bytes = reads * 8.0 / 14e6;   // us per position and dim
-    const double rows_us = (double)q_len * seen * (double)head_dim * (by_macs > by_bytes ? by_macs : by_bytes);
-    return rows_us > 1.2 * (12.0 + (double)kv_len * (double)(n_head_kv * head_dim) * 8.0 / 3.5e6);
-}
-
 // Launch plan: whole tiles, or pieces of `chunk` position blocks (partial
 // states merged by attn_combine_few_kernel).  The plan assumes the chunk's queries are the
 // last q_len of the kv_len positions (a prompt); at launch only the piece
@@ -62,6 +36,7 @@ struct ApPlan {
     int tiles;    // per group
     int chunk;    // position blocks per piece; 0: whole tiles, no partial states
     int stride;   // partial states per (query row, head)
+    double us;    // expected time of the kernel and the merge (0: whole tiles, two or more workgroups per CU)
 };
 
 // A launch's time, us, if the tiles (runs of equal length, shortest first) are
@@ -133,12 +108,13 @@ inline ApPlan ap_plan(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q
     int chunk = longest;
     if (pieces > 0) {
         chunk = (longest + pieces - 1) / pieces;
+        p.us = ap_time(runs, (size_t)p.groups, head_dim, cus, chunk);
     } else {
         // Candidates: the smallest chunks that leave at most 1/4, 1/2, ... 2, 2
         // 1/2, ... 4 pieces per CU (more never measured faster).  Smaller chunks of as many
         // rounds of pieces only add pieces to merge, larger ones make the pieces
         // longer.  Ties keep the larger chunk.
-        double best = ap_time(runs, (size_t)p.groups, head_dim, cus, longest);
+        double best = p.us = ap_time(runs, (size_t)p.groups, head_dim, cus, longest);
         for (int k = 1; k <= 16; k += k < 8 ? 1 : 2) {
             const size_t most = cus * (size_t)k / 4 / (size_t)p.groups;   // per head group
             if (most <= (size_t)p.tiles) continue;
@@ -156,7 +132,7 @@ inline ApPlan ap_plan(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q
             if (lo >= chunk) continue;
             const double e = ap_time(runs, (size_t)p.groups, head_dim, cus, lo);
             if (e < best - 1e-9) {
-                best = e;
+                best = p.us = e;
                 chunk = lo;
             }
         }
@@ -167,6 +143,43 @@ inline ApPlan ap_plan(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q
     p.chunk = chunk;
     p.stride = (nbmax + chunk - 1) / chunk;
     return p;
+}
+
+// Expected time, us, of the decode kernel (attention.hip), which runs each
+// query row by itself: its products at 4.8 Tera multiply-adds/s (QK and PV
+// counted once; up to 30 % more of them for many rows), or its K and V rows,
+// read once per kv head for groups of 2, 4 or 8 query heads, else once per query
+// head, at 11.5 TB/s, or 31 TB/s when the layer's K and V are below 8 MB and
+// stay in the L2s.
+inline double ap_rows_time(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len) {
+    const size_t g = n_head_kv && n_head % n_head_kv == 0 ? n_head / n_head_kv : 1;
+    const double reads = (double)(g == 2 || g == 4 || g == 8 ? n_head_kv : n_head);   // of K and V per query row
+    const double seen = (double)kv_len - 0.5 * (double)(q_len < kv_len ? q_len : kv_len);
+    const double by_macs = (double)n_head / 4.8e6 * (q_len > 8 ? 0.7 + 2.4 / (double)q_len : 1.0);
+    const double by_bytes = reads * 8.0 / ((double)kv_len * (double)(n_head_kv * head_dim) * 8.0 < 8e6 ? 31e6 : 11.5e6);
+    return 10.0 + (double)q_len * seen * (double)head_dim * (by_macs > by_bytes ? by_macs : by_bytes);
+}
+
+// Whether a chunk takes this kernel: head_dim 64 or 128, a kv head's rows
+// addressable by the 32-bit buffer offsets of its K/V loads, and clearly less
+// time expected than for the decode kernel; this one's launches cost 9.4 us
+// beside ap_time.  Fitted on MI355X to both kernels' times at 560 calls (14 head
+// counts, both dims, 2 to 512 rows, 0 to 16000 cached): the kernel it takes is
+// 2.6 % slower than the faster one on average (always this one 8 %, always the
+// decode kernel 145 %), and this one is taken where it is over 10 % slower in 3
+// of them (without the factor 1.1 in 12).  Some calls, us, decode kernel / this
+// one: 32/8 heads of 128, 4000 cached, 6 / 8 / 12 rows 25 / 31, 31 / 31, 44 / 33;
+// 500 cached, 48 / 64 rows 23 / 24, 23 / 25; from position 0, 64 / 203 rows 7 /
+// 17, 21 / 23; 32/8 heads of 64, 4000 cached, 8 / 12 rows 19 / 21, 25 / 22; 32/32
+// heads of 128, 4000 cached, 4 / 6 rows 48 / 43, 70 / 43; 14/2 heads of 64, 4000
+// cached, 8 rows 16 / 20.  (BARQ_ATTN_MFMA_MIN_Q: this kernel from that many
+// rows on, whatever the times.)
+inline bool ap_supported(size_t head_dim, size_t kv_len) {
+    return (head_dim == 64 || head_dim == 128) && kv_len < ((size_t)1 << 23);
+}
+inline bool ap_path(size_t n_head, size_t n_head_kv, size_t head_dim, size_t q_len, size_t kv_len, const ApPlan& plan) {
+    return ap_supported(head_dim, kv_len) && q_len >= 2 &&
+           ap_rows_time(n_head, n_head_kv, head_dim, q_len, kv_len) > 1.1 * (9.4 + plan.us);
 }
 
 }  // namespace barq
