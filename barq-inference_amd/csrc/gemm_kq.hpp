@@ -498,6 +498,12 @@ __device__ __forceinline__ void kq_step(uint8_t* const (&stages)[KQ_MAX_NS], int
     if (b + NS - 1 < nst)
         kq_issue<F, BM, NW>(stages[(S + NS - 1) % NS] + sub, xr, wr, off, KG * (b + NS - 1) + kg, wave);
     kq_compute<F, BM, NW>(stages[S] + sub, KG * b + kg, wave, l, acc);
+    if constexpr (BM == 128)
+        // with two chains: the sums here and not, with the integer sums kept until then, where the chain goes on
+        #pragma unroll
+        for (int t = 0; t < L::MTW; t++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++) asm volatile("" : "+v"(acc[t][r]));
 }
 
 // The Q4_K two-K-group step with group 1's epilogue deferred: group 0 runs
@@ -545,11 +551,13 @@ __device__ __forceinline__ void kq4_round_defer(std::integer_sequence<int, S...>
 // at X (row bytes xrb) against weight rows [n0, n0 + 128) of W; results to
 // Y[row * N + col].  All waves of the workgroup call it with the same values.
 // NS consecutive steps (one per stage), unrolled so that stage indices are constants
-template <class F, int BM, int NW, int NS, int KG, int... S>
+// (with two chains, super-block b adds to chain b % 2)
+template <class F, int BM, int NW, int NS, int KG, int CH, int... S>
 __device__ __forceinline__ void kq_round(std::integer_sequence<int, S...>, uint8_t* const (&stages)[KQ_MAX_NS], int b,
                                          int nst, i32x4v xr, i32x4v wr, const KQOff<F, BM, NW>& off, int kg, int wave,
-                                         int l, float (&acc)[KQL<F, BM, NW>::MTW][16]) {
-    (kq_step<F, BM, NW, NS, KG, S>(stages, b + S, nst, xr, wr, off, kg, wave, l, acc), ...);
+                                         int l, float (&acc)[CH][KQL<F, BM, NW>::MTW][16]) {
+    static_assert(NS % CH == 0, "a stage's super-blocks belong to one chain");
+    (kq_step<F, BM, NW, NS, KG, S>(stages, b + S, nst, xr, wr, off, kg, wave, l, acc[S % CH]), ...);
 }
 
 // Tile results to Y[row * N + col] for rows < count and columns < N, with
@@ -626,11 +634,19 @@ __device__ __forceinline__ void kq_tile(uint8_t* const (&stages)[KQ_MAX_NS], con
     const i32x4v xr = make_rsrc4(X + (size_t)m0 * xrb + xk, (uint32_t)((size_t)(count - m0) * xrb) - xk);
     const i32x4v wr = make_rsrc4(W + (size_t)n0 * wrb + wk, (uint32_t)((size_t)(N - n0) * wrb) - wk);
 
-    float acc[MT][16];
+    // The 128-row tiles have one K-group and two chains of f32 sums, even and
+    // odd super-blocks, added at the end: the sums of two K-groups, bit for bit
+    // (error against 64 bits at k = 4096 / 14336 8.1e-8 / 1.14e-7; one chain
+    // 9.2e-8 / 1.46e-7).  Times are those of one chain.
+    constexpr int CH = BM == 128 && KG == 1 && NS % 2 == 0 ? 2 : 1;
+    float chains[CH][MT][16];
     #pragma unroll
-    for (int t = 0; t < MT; t++)
+    for (int h = 0; h < CH; h++)
         #pragma unroll
-        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+        for (int t = 0; t < MT; t++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++) chains[h][t][r] = 0.0f;
+    float (&acc)[MT][16] = chains[0];
 
     KQOff<F, BM, NW> off;
     kq_offsets<F, BM, NW>(off, xrb, wrb, wave, l);
@@ -647,10 +663,16 @@ __device__ __forceinline__ void kq_tile(uint8_t* const (&stages)[KQ_MAX_NS], con
         if (kg == 1 && nst > 0) kq4_epilogue<MT>(part, dxs, acc);
     } else {
         for (int b = 0; b < nst; b += NS)
-            kq_round<F, BM, NW, NS, KG>(std::make_integer_sequence<int, NS>{}, stages, b, nst, xr, wr, off, kg, wave,
-                                        l, acc);
+            kq_round<F, BM, NW, NS, KG, CH>(std::make_integer_sequence<int, NS>{}, stages, b, nst, xr, wr, off, kg, wave,
+                                            l, chains);
     }
 
+    if constexpr (CH == 2) {
+        #pragma unroll
+        for (int t = 0; t < MT; t++)
+            #pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] += chains[1][t][r];
+    }
     if constexpr (KG > 1) kq_reduce_groups<F, BM, NW, KG>(stages[0], acc, kg, wave, l);
     if (kg == 0) kq_store<F, BM, NW>(acc, Y, count, N, m0, n0, wave, l);
 }

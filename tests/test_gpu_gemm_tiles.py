@@ -92,3 +92,14 @@ def test_expert_gather_of_more_blocks_than_workgroups(be):
                       B.ACT_F32_Q8).cpu().numpy() for b in (be, two)]
     two.close()
     assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("n,k,m", [(16500, 512, 65), (16512, 4096, 128), (11000, 1024, 193)])
+def test_q4_k_128_row_tiles_sum_like_64_row_ones(be, n, k, m):
+    """Two chains of f32 sums (even and odd super-blocks) on both: the same bits."""
+    w, x = synth.gen_q4_k(n, k, 3), synth.gen_f32(m * k, 4).reshape(m, k)
+    xq = be.quantize_act(B.Q8_K, dev(x))
+    small = backend(BARQ_GEMM_BM="64")
+    outs = [b.matmul(B.Q4_K, dev(w), n, k, B.Q8_K, xq, m).cpu().numpy() for b in (be, small)]
+    small.close()
+    assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
