@@ -412,20 +412,24 @@ static hipError_t b32_launch_t(const void* W, size_t n_rows, size_t k, const int
 
 // More 64-row tiles than CUs: one K-group of four waves per workgroup, so that
 // two or three workgroups share a CU and a last round that leaves CUs without
-// a tile costs less; fewer than two tiles per CU are cut into 32-row ones.
-// Measured on MI355X, us per call with the repack, for 64-row tiles with two
-// K-groups (one workgroup per CU) / 64-row / 32-row tiles with one, two
-// stages each: Q8_0 6144 x 4096, M = 333 (288 tiles, f32 rows) 70.9 / 62.3 /
-// 58.8; Q4_0 the same 66.5 / 54.1 / 48.9; Q4_0 14336 x 4096, M = 512 (896)
-// 131 / 99 / 107 (118 / 125 with three stages, which leave room for two
-// workgroups instead of three); Q4_0 9000 x 5120, M = 700 (781) 166 / 122 /
-// 137; with a tile per CU (Q4_0 4096 x 4096, M = 512) 38.0 / 45.7 / 40.1.
+// a tile costs less; cut into 32-row tiles while those are at most three per
+// CU, which then run at once.  Measured on MI355X, us per call with the repack,
+// for 64-row tiles with two K-groups (one workgroup per CU) / 64-row / 32-row
+// tiles with one, two stages each, k = 4096: Q8_0, 288 / 320 / 384 tiles of 64
+// rows 70 / 70 / 57, 73 / 72 / 61, 70 / 68 / 60; 400 / 448 / 512 tiles - / 75 /
+// 83, 69 / 68 / 79, 70 / 69 / 79; Q4_0, 288 / 320 / 384 68 / 62 / 49, 72 / 68 /
+// 60, 70 / 66 / 57; 400 / 448 / 512 - / 64 / 64, 69 / 65 / 67, 70 / 65 / 69;
+// Q4_0 14336 x 4096, M = 512 (896) 131 / 99 / 107 (118 / 125 with three stages,
+// which leave room for two workgroups instead of three); with a tile per CU
+// (Q4_0 4096 x 4096, M = 512) 38.0 / 45.7 / 40.1.  Up to 32 rows, two K-groups /
+// one: Q8_0 128256 x 4096, M = 4 / 16 / 32 120 / 118, 137 / 133, 139 / 138;
+// 40000 x 4096, M = 16 65 / 52; Q4_0 91 / 89, 103 / 85, 104 / 88; 49 / 39.
 static bool b32_many_tiles(size_t m, size_t n_rows) {
-    return (m + 63) / 64 * ((n_rows + B32_BN - 1) / B32_BN) > 256;
+    return (m + 63) / 64 * ((n_rows + B32_BN - 1) / B32_BN) > (size_t)cu_count_attn();
 }
 
 static int b32_bm(size_t m, size_t n_rows) {
-    const bool few = b32_many_tiles(m, n_rows) && (m + 63) / 64 * ((n_rows + B32_BN - 1) / B32_BN) < 512;
+    const bool few = b32_many_tiles(m, n_rows) && (m + 31) / 32 * ((n_rows + B32_BN - 1) / B32_BN) <= 3 * (size_t)cu_count_attn();
     const int bm = tuning_env(TUNE_GEMM_BM, m > 32 && !few ? 64 : 32);
     return bm == 32 ? 32 : 64;
 }

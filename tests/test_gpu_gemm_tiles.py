@@ -46,7 +46,10 @@ def test_expert_groups_of_64_row_tiles(be, rows):
 @pytest.mark.parametrize("t", [B.Q4_0, B.Q8_0, B.Q4_0_BARQ])
 @pytest.mark.parametrize("n,m,scale", [
     (16400, 65, 1.0),     # 258 tiles of 64 rows: 32-row tiles, one K-group
+    (17000, 192, 1.0),    # 399 tiles of 64 rows, more than three of 32 rows per CU: 64-row tiles, one K-group
     (21800, 130, 1.0),    # 513 tiles: 64-row tiles, one K-group
+    (32800, 4, 1.0),      # more tiles than CUs for a few rows: 32-row tiles, one K-group
+    (32800, 32, 1.0),
     (200, 70, 1e-6),      # activation scales that are subnormal in f16
     (200, 33, 3e4),       # large ones
 ])
