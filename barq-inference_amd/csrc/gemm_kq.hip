@@ -67,7 +67,7 @@ static hipError_t kq_dispatch(const KQArgs& a, size_t rows, hipStream_t s) {
     const int g_kq_ns = tuning_env(TUNE_GEMM_NS), g_kq_bm = tuning_env(TUNE_GEMM_BM);
     const int bm = g_kq_bm ? g_kq_bm
                  : (!GROUPED && F::TYPE == TYPE_Q6_K && kq6_wide_tiles(rows, (size_t)a.N, (size_t)a.nsb)) ? 66
-                 : (rows > (GROUPED ? 40 : 32) ? 64 : 32);
+                 : (rows > (GROUPED ? 31 : 32) ? 64 : 32);
     if (bm == 16) {
         if (g_kq_ns == 2) return kq_launch_t<F, 16, 2, 4, GROUPED>(a, s);
         if (g_kq_ns == 4) return kq_launch_t<F, 16, 4, 4, GROUPED>(a, s);
@@ -108,14 +108,16 @@ static hipError_t kq_dispatch(const KQArgs& a, size_t rows, hipStream_t s) {
         }
     }
     if constexpr (GROUPED) {
-        // Expert groups of more than 40 rows: 64-row tiles of four waves of
-        // 64 x 32, so that a wave decodes its weights once for two MFMA row
-        // tiles; two stages (two workgroups per CU for Q4_K).  Measured on
-        // MI355X, Mixtral-8x7B shapes, top-2 of 8 experts, us per expert FFN
-        // of 64 / 128 / 200 / 256 / 512 tokens: 289 / 303 / 378 / 437 / 756;
-        // 32-row tiles 225 / 287 / 416 / 471 / 830; eight waves of 32 x 32 on
-        // 64-row tiles (each weight decoded twice per tile) 234 / 298 / 446 /
-        // 524 / 889.
+        // Expert groups of 32 rows or more on average: 64-row tiles of four
+        // waves of 64 x 32, so that a wave decodes its weights once for two MFMA
+        // row tiles; two stages (two workgroups per CU for Q4_K).  Measured on
+        // MI355X, Mixtral-8x7B shapes, top-2 of 8 experts, us per expert FFN of
+        // 112 / 124 / 128 / 136 / 160 / 200 / 256 / 512 tokens: 310 / 312 / 314 /
+        // 321 / 324 / 378 / 437 / 756; 32-row tiles 279 / 309 / 348 / 353 / 366 /
+        // 416 / 471 / 830; eight waves of 32 x 32 on 64-row tiles (each weight
+        // decoded twice per tile) - / - / - / 369 / 378 / 446 / 524 / 889.  The two
+        // cross between 31 and 32 rows, where half the groups need a second
+        // 32-row tile, at 2048 x 4096, 4096 x 4096 and 3072 x 8192 too.
         if (bm >= 64) return kq_launch_t<F, 64, 2, 4, GROUPED>(a, s);
     }
     if constexpr (F::TYPE == TYPE_Q4_K) {

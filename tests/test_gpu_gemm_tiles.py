@@ -25,9 +25,9 @@ def backend(**env):
             os.environ.pop(k) if v is None else os.environ.__setitem__(k, v)
 
 
-@pytest.mark.parametrize("rows", [41, 63, 64, 65, 129])
+@pytest.mark.parametrize("rows", [31, 32, 33, 41, 63, 64, 65, 129])
 def test_expert_groups_of_64_row_tiles(be, rows):
-    """Expert groups above 40 rows take 64-row tiles; a weight row's products
+    """Expert groups of 32 rows or more take 64-row tiles; a weight row's products
     are summed in the same order as on 32-row tiles, so the outputs are the
     same bits.  Three experts with `rows` - 20, `rows` and `rows` + 20 rows."""
     hidden, n_ff, ne = 512, 768, 3
