@@ -135,19 +135,20 @@ ATTN_CASES = [
     (4, 2, 64, 16, 16, 0, 16),            # a prompt from position 0
     (8, 2, 128, 3, 10, 2, 10),            # start_pos + q_len < kv_len: masked tail
     (8, 2, 128, 1, 50, 49, 80),           # kv_len below the layer length
-    # prompt chunks of 32+ rows (head_dim 128: the MFMA kernel)
-    (32, 8, 128, 32, 32, 0, 32),          # one query block from position 0
-    (32, 8, 128, 100, 150, 50, 160),      # ragged last block, chunk after a prefix
+    # prompt chunks (on whichever kernel the work of the call takes; all of them
+    # on the prompt kernel in test_prompt_cases_on_the_prompt_kernel)
+    (32, 8, 128, 32, 32, 0, 32),          # one block of positions
+    (32, 8, 128, 100, 150, 50, 160),      # ragged last tile, chunk after a prefix
     (8, 2, 128, 64, 64, 0, 64),
     (12, 6, 128, 40, 300, 260, 300),      # 2 per kv head
     (6, 4, 128, 33, 33, 0, 40),           # irregular grouping
     (8, 2, 128, 40, 100, 20, 100),        # start_pos + q_len < kv_len: masked tail
     (32, 8, 128, 512, 512, 0, 512),       # a Llama-3-8B prompt of 512 tokens
-    (32, 8, 128, 768, 768, 0, 768),       # pieces of 6 position blocks, two workgroups per CU
-    (32, 8, 128, 200, 1000, 800, 1000),   # a chunk after a long prefix: every query block in pieces
-    (4, 2, 64, 48, 48, 0, 48),            # head_dim 64 stays on the split kernel
-    (32, 32, 128, 512, 512, 0, 512),      # query blocks paired (long + short) per workgroup
-    (64, 64, 128, 288, 300, 12, 300),     # paired, odd block count (the middle block alone)
+    (32, 8, 128, 768, 768, 0, 768),       # in pieces
+    (32, 8, 128, 200, 1000, 800, 1000),   # a chunk after a long prefix: every tile in pieces
+    (4, 2, 64, 48, 48, 0, 48),
+    (32, 32, 128, 512, 512, 0, 512),      # one query head per kv head
+    (64, 64, 128, 288, 300, 12, 300),
 ]
 
 
@@ -172,6 +173,35 @@ def test_attention_matches_oracle(be, orc, n_head, n_kv, hd, q_len, kv_len, star
     assert err <= 2e-5 * np.max(np.abs(v)), err
     host = A.compute_attention(be, q, c, 1, n_head, n_kv, hd, q_len, kv_len, start, mem=B.MEM_HOST)
     assert np.array_equal(host, got)
+    c.close()
+
+
+def prompt_backend(pieces=0):
+    """A handle whose chunks of any length run the prompt kernel, every tile in
+    at least `pieces` pieces of the longest one's (0: the plan's)."""
+    import os
+    env = {"BARQ_ATTN_MFMA_MIN_Q": "1", "BARQ_ATTN_MFMA_SPLIT": str(pieces)}
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update(env)
+    try:
+        return B.Backend(0)
+    finally:
+        for k, v in old.items():
+            os.environ.pop(k) if v is None else os.environ.__setitem__(k, v)
+
+
+@pytest.mark.parametrize("n_head,n_kv,hd,q_len,kv_len,start,pos", [c for c in ATTN_CASES if c[3] > 1 and c[2] < 256])
+def test_prompt_cases_on_the_prompt_kernel(be, orc, n_head, n_kv, hd, q_len, kv_len, start, pos):
+    c, k, v = fill_cache(be, n_kv, hd, pos, n_head * 7 + kv_len)
+    q = rng_f32(kv_len + 3, n_head, q_len, hd)
+    be.sync()
+    ref = orc.attention(q, k, v, n_head, q_len, kv_len, start)
+    for pieces in (0, 2):
+        b = prompt_backend(pieces)
+        got = A.compute_attention(b, dev(q), c, 1, n_head, n_kv, hd, q_len, kv_len, start).cpu().numpy()
+        b.close()
+        err = np.max(np.abs(got - ref))
+        assert err <= 2e-5 * np.max(np.abs(v)), (pieces, err)
     c.close()
 
 
@@ -229,7 +259,9 @@ def test_append_rope_q_equals_separate_steps(be, layout, n_head, n_kv, hd, n):
     (32, 8, 128, 1, 4096, 4095, 4096),    # decode: the merge writes Q8_K blocks
     (32, 8, 128, 1, 40, 39, 40),          # one split: attention, then the quantizer
     (32, 8, 128, 7, 300, 293, 300),       # a chunk of 7 rows
-    (32, 8, 128, 40, 100, 60, 100),       # a prompt chunk on the MFMA kernel
+    (32, 8, 128, 40, 100, 60, 100),       # a prompt chunk on the decode kernel
+    (32, 8, 128, 100, 1000, 900, 1000),   # a prompt chunk on the prompt kernel: its merge writes the blocks
+    (32, 8, 64, 100, 2000, 1900, 2000),   # four heads per block
     (8, 2, 64, 1, 1000, 999, 1000),       # head_dim 64: four heads per block
     (4, 2, 256, 1, 517, 516, 517),        # head_dim 256: one head per block
     (8, 1, 64, 1, 20000, 19999, 20000),   # 157 splits (test_attention_q8k_many_splits: more than the merge's threads)
@@ -249,16 +281,17 @@ def test_attention_q8k_equals_quantized_attention(be, n_head, n_kv, hd, q_len, k
     c.close()
 
 
-def test_attention_prompt_pieces_random_shapes(be, orc):
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("pieces", [0, 2, 5])
+def test_attention_prompt_pieces_random_shapes(be, orc, hd, pieces):
     """Prompt chunks of seeded random lengths after random cached prefixes
-    (some with a masked tail: start_pos + q_len < kv_len) on the MFMA prompt
-    kernel, whose pieces per query block follow the launch simulation's chunk:
-    the f32 rows against the oracle, and the Q8_K merge against quantizing
-    them."""
+    (some with a masked tail: start_pos + q_len < kv_len) on the prompt kernel,
+    cut as the plan has it and the longest tile into two and five pieces: the
+    f32 rows against the oracle, and the Q8_K merge against quantizing them."""
     rng = np.random.default_rng(2024)
+    b = prompt_backend(pieces)
     for case in range(10):
         n_head, n_kv = [(8, 2), (12, 6), (16, 4), (32, 8)][case % 4]
-        hd = 128
         q_len = int(rng.integers(32, 200))
         prefix = int(rng.integers(0, 400))
         kv_len = prefix + q_len
@@ -267,15 +300,17 @@ def test_attention_prompt_pieces_random_shapes(be, orc):
               f"start={start}", flush=True)
         c, k, v = fill_cache(be, n_kv, hd, kv_len, 900 + case)
         q = rng_f32(950 + case, n_head, q_len, hd)
-        y = A.compute_attention(be, dev(q), c, 1, n_head, n_kv, hd, q_len, kv_len, start)
+        be.sync()
+        y = A.compute_attention(b, dev(q), c, 1, n_head, n_kv, hd, q_len, kv_len, start)
         ref = orc.attention(q, k, v, n_head, q_len, kv_len, start)
         err = np.max(np.abs(y.cpu().numpy() - ref))
         assert err <= 2e-5 * np.max(np.abs(v)), (case, err)
         if (n_head * hd) % 256 == 0:
-            q8 = A.compute_attention_q8k(be, dev(q), c, 1, n_head, n_kv, hd, q_len, kv_len, start)
-            want = be.quantize_act(B.Q8_K, y.reshape(q_len, n_head * hd)).cpu().numpy().reshape(-1)
+            q8 = A.compute_attention_q8k(b, dev(q), c, 1, n_head, n_kv, hd, q_len, kv_len, start)
+            want = b.quantize_act(B.Q8_K, y.reshape(q_len, n_head * hd)).cpu().numpy().reshape(-1)
             assert np.array_equal(q8.cpu().numpy().reshape(-1), want), case
         c.close()
+    b.close()
 
 
 def test_attention_q8k_argument_errors(be):
@@ -287,14 +322,14 @@ def test_attention_q8k_argument_errors(be):
 
 
 @pytest.mark.parametrize("n_head,n_kv,q_len,kv_len,start,pos", [
-    (32, 8, 1, 300, 299, 300),    # a decode row on the MFMA kernel
-    (32, 8, 7, 40, 33, 40),       # a short chunk: one block, 25 rows unused
+    (32, 8, 1, 300, 299, 300),    # a decode row on the prompt kernel
+    (32, 8, 7, 40, 33, 40),       # a short chunk: one tile, 100 rows unused
     (8, 2, 16, 16, 0, 16),
     (12, 6, 3, 10, 2, 10),        # masked tail
 ])
 def test_attention_mfma_kernel_small_chunks(be, orc, n_head, n_kv, q_len, kv_len, start, pos):
-    """The MFMA prompt kernel with its threshold lowered (BARQ_ATTN_MFMA_MIN_Q,
-    read at handle creation) on chunks shorter than a query block."""
+    """The prompt kernel with its threshold lowered (BARQ_ATTN_MFMA_MIN_Q, read
+    at handle creation) on chunks shorter than a tile."""
     import os
     hd = 128
     c, k, v = fill_cache(be, n_kv, hd, pos, n_head * 5 + kv_len)

@@ -5,8 +5,9 @@ finite, and the rule that chooses it.  Parity against the oracle
 
 Bar: 2e-5 of the largest |V| of the same output dim.  Outputs are convex
 combinations of V rows, and a score is a dot product of 64 or 128 terms, each
-to 2^-24 of |q||k|, so at the sizes here (|score| below 10) a weight is off by
-less than 10 * 2^-22 and an output by less than 1e-5 of the largest |V|.
+to 2^-22 of its |q||k| (two values split to 2^-23 each, their small parts'
+product left out), so at the sizes here (|score| below 10) a weight is off by
+less than 10 * 2^-21 and an output by less than 1e-5 of the largest |V|.
 """
 import os
 
@@ -88,7 +89,8 @@ def test_tile_edges(prompt_be, orc, hd, n_head, n_kv, q_len, start, kv_len):
 @pytest.mark.parametrize("hd", [64, 128])
 def test_value_ranges(prompt_be, orc, hd):
     """Scales per position (K), per query row (Q) and per dim (V, growing with
-    the positions, one dim zero for two blocks, one zero throughout)."""
+    the positions by up to 2^20, one dim zero for two blocks, one zero
+    throughout)."""
     n_head, n_kv, q_len, kv_len = 8, 2, 100, 200
     r = np.random.default_rng(hd)
     q, k, v = (r.standard_normal(s) for s in ((n_head, q_len, hd), (n_kv, kv_len, hd), (n_kv, kv_len, hd)))
@@ -99,7 +101,7 @@ def test_value_ranges(prompt_be, orc, hd):
     v[:, :, 5] = 0
     q, k, v = q.astype(F32), k.astype(F32), v.astype(F32)
     out = attend(prompt_be, q, k, v, kv_len - q_len, n_head)
-    # a row's results only depend on what it sees: the bar per row uses V up to it
+    # the bar per row uses V up to it (test_values_beside_a_large_one: what it does not see)
     ref = orc.attention(q, k, v, n_head, q_len, kv_len, kv_len - q_len)
     for i in (0, 40, q_len - 1):
         close(out[i:i + 1], ref[i:i + 1], v[:, :kv_len - q_len + i + 1], n_head)
