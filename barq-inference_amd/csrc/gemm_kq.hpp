@@ -498,7 +498,7 @@ __device__ __forceinline__ void kq_step(uint8_t* const (&stages)[KQ_MAX_NS], int
     if (b + NS - 1 < nst)
         kq_issue<F, BM, NW>(stages[(S + NS - 1) % NS] + sub, xr, wr, off, KG * (b + NS - 1) + kg, wave);
     kq_compute<F, BM, NW>(stages[S] + sub, KG * b + kg, wave, l, acc);
-    if constexpr (BM == 128)
+    if constexpr (F::TYPE == TYPE_Q4_K && BM == 128)
         // with two chains: the sums here and not, with the integer sums kept until then, where the chain goes on
         #pragma unroll
         for (int t = 0; t < L::MTW; t++)
@@ -634,11 +634,11 @@ __device__ __forceinline__ void kq_tile(uint8_t* const (&stages)[KQ_MAX_NS], con
     const i32x4v xr = make_rsrc4(X + (size_t)m0 * xrb + xk, (uint32_t)((size_t)(count - m0) * xrb) - xk);
     const i32x4v wr = make_rsrc4(W + (size_t)n0 * wrb + wk, (uint32_t)((size_t)(N - n0) * wrb) - wk);
 
-    // The 128-row tiles have one K-group and two chains of f32 sums, even and
+    // The 128-row Q4_K tiles have one K-group and two chains of f32 sums, even and
     // odd super-blocks, added at the end: the sums of two K-groups, bit for bit
     // (error against 64 bits at k = 4096 / 14336 8.1e-8 / 1.14e-7; one chain
     // 9.2e-8 / 1.46e-7).  Times are those of one chain.
-    constexpr int CH = BM == 128 && KG == 1 && NS % 2 == 0 ? 2 : 1;
+    constexpr int CH = F::TYPE == TYPE_Q4_K && BM == 128 && KG == 1 && NS % 2 == 0 ? 2 : 1;
     float chains[CH][MT][16];
     #pragma unroll
     for (int h = 0; h < CH; h++)

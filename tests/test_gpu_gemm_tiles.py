@@ -106,3 +106,14 @@ def test_q4_k_128_row_tiles_sum_like_64_row_ones(be, n, k, m):
     outs = [b.matmul(B.Q4_K, dev(w), n, k, B.Q8_K, xq, m).cpu().numpy() for b in (be, small)]
     small.close()
     assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
+
+
+def test_q6_k_128_row_tiles_sum_like_64_row_ones(be):
+    """One chain of f32 sums on both (no K slices at this width): the same bits."""
+    n, k, m = 16512, 1024, 256
+    w, x = synth.gen_q6_k(n, k, 3), synth.gen_f32(m * k, 4).reshape(m, k)
+    xq = be.quantize_act(B.Q8_K, dev(x))
+    small = backend(BARQ_GEMM_BM="66")
+    outs = [b.matmul(B.Q6_K, dev(w), n, k, B.Q8_K, xq, m).cpu().numpy() for b in (be, small)]
+    small.close()
+    assert np.any(outs[0]) and np.array_equal(outs[0], outs[1])
