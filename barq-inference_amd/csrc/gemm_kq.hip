@@ -52,6 +52,7 @@ static bool kq6_tall_tiles(size_t m, size_t n_rows, size_t nsb) {
 static bool kq4_tall_tiles(size_t m, size_t n_rows) {
     const int bm_env = tuning_env(TUNE_GEMM_BM);
     if (bm_env) return bm_env == 68;
+    if (tuning_env(TUNE_GEMM_NS) || tuning_env(TUNE_GEMM_KG) || tuning_env(TUNE_GEMM_DEFER, 3) != 3) return false;   // of the 64-row tiles
     const size_t tiles_n = (n_rows + KQ_BN - 1) / KQ_BN, cus = (size_t)cu_count();
     const auto rounds = [&](size_t bm) { return ((m + bm - 1) / bm * tiles_n + cus - 1) / cus; };
     return rounds(64) >= 2 * rounds(128);
