@@ -52,11 +52,14 @@
 //
 // Measured on MI355X, us per call with the merge (the f32-MFMA kernel for 128
 // dims, the decode kernel for 64, before this one): Llama-3-8B heads, 2048 /
-// 1024 / 512 / 256 tokens 210 / 71 / 40 / 25.6 against 337 / 135 / 54 / 30;
+// 1024 / 512 / 256 tokens 206 / 73 / 40 / 26 against 337 / 135 / 54 / 30;
 // 200 rows after 800 with heads of 64 dims 26 against 55.  (With lo as it is,
 // one scale per row for P and no look at V's spread: 190 / 68 / 37 / 24 / 25.
 // P V on f32 MFMAs: 317 / 100 / 48 / 27 / 28.)  Error against 64 bits (relative
-// 2-norm, the same calls) 1.6e-7 to 1.9e-7 against 2.0e-7 to 3.9e-7.
+// 2-norm, the same calls) 1.5e-7 to 1.9e-7 against 2.0e-7 to 3.9e-7.  At 2048
+// tokens the matrix unit is 23 % busy and vector issue 31 % (524 vector
+// instructions besides the 48 MFMAs per wave and block): a wave's scores,
+// weights and output follow one another, and two waves share a SIMD.
 #include "attention_prompt_plan.hpp"
 #include "common.hpp"
 #include "launch.hpp"
@@ -80,8 +83,7 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // of row i; fewer in a last wave), four values per lane; Q8, whose rows are
 // whole blocks, writes the values' Q8_K block (q8_k_block) instead of them.  One pass over
 // the pieces, each rescaling what was summed before it, so a row waits for
-// memory once per two pieces and not twice per piece (2048 tokens in two
-// pieces per long tile: see attn_prompt_plan).
+// memory once per two pieces and not twice per piece.
 template <int HD, bool Q8>
 __global__ __launch_bounds__(256)
 void attn_combine_few_kernel(const float* __restrict__ part, int stride, int chunk, int n_head, int G, int q_len,
