@@ -292,3 +292,32 @@ def test_heads_of_no_whole_q8_k_blocks(orc, monkeypatch, hd, n_head, n_kv, q_len
     out = attend_f32(b, q, k, v, n_head)
     b.close()
     close(out, orc.attention(q, k, v, n_head, q_len, kv_len, start), v, n_head)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("pieces", [0, 2])
+def test_outputs_at_any_float(orc, monkeypatch, hd, pieces):
+    """The output need only be 4-byte aligned; what stands around it stays."""
+    import torch
+    if pieces:
+        monkeypatch.setenv("BARQ_ATTN_MFMA_SPLIT", str(pieces))
+    b = backend(1)
+    n_head, n_kv, q_len, kv_len = 6, 2, 50, 100
+    r = np.random.default_rng(hd)
+    q, k, v = (r.standard_normal(s).astype(F32) for s in ((n_head, q_len, hd), (n_kv, kv_len, hd), (n_kv, kv_len, hd)))
+    c = A.KVCache(b, kv_len, 1, n_kv, hd)
+    c.append(0, k, v, kv_len, hd, mem=B.MEM_HOST)
+    n = q_len * n_head * hd
+    buf, qd = torch.full((n + 8,), 7.0, device="cuda"), dev(q)
+    torch.cuda.synchronize()
+    for at in (1, 2, 3):
+        buf.fill_(7.0)
+        torch.cuda.synchronize()
+        B._lib.check(b._lib.barq_rocm_attention(b.h, qd.data_ptr(), c.c, 0, n_head, n_kv, hd, q_len, kv_len, kv_len - q_len,
+                                                buf.data_ptr() + 4 * at, B.MEM_DEVICE))
+        b.sync()
+        got = buf.cpu().numpy()
+        assert np.all(got[:at] == 7.0) and np.all(got[at + n:] == 7.0)
+        close(got[at:at + n].reshape(q_len, n_head, hd), orc.attention(q, k, v, n_head, q_len, kv_len, kv_len - q_len), v, n_head)
+    c.close()
+    b.close()
