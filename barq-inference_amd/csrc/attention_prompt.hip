@@ -17,7 +17,7 @@
 // rate (157 TFLOP/s against 2.5 PFLOP/s), and a kernel on it ran at 105
 // TFLOP/s.  Here every f32 operand x is scaled by a power of two and split
 // into two f16 values, each rounded to nearest: x = hi + lo + e with |e| <=
-// 2^-23 |x| (2^-25 root mean square; three quarters of all mantissas split
+// 2^-23 |x| (2^-24.5 root mean square; three quarters of all mantissas split
 // exactly), and a product takes three f16 MFMAs (hi hi, hi lo, lo hi; lo lo is
 // at most 2^-22 of it, 2^-24.6 root mean square) with f32 sums, 5.3 times the
 // f32 rate.  Scales keep the split away from f16's limits:
@@ -37,12 +37,13 @@
 // Weights and values spread further (a first position that takes nearly all
 // the weight; a large value that a row does not see), and what they lose is
 // not small against the result when the large ones add little to it.  lo of P
-// and V is held times 2^11, so that its steps end at 2^-35: weights down to
-// 2^-26 of their block's largest (18 nats) and values down to 2^-25 keep all
-// bits.  Weights further down lose one per halving (in that block alone); a
-// tile with values below 2^-34 of their dim's scale, or with a scale that
-// shrinks by more than that, goes to ap_rows_f32 too, and so does one whose
-// sums are not finite (infinities and NaN turn into NaN here).
+// and V is held times 2^12, so that its steps end at 2^-36: weights down to
+// 2^-27 of their block's largest (19 nats) and values down to 2^-26 of their
+// dim's keep all bits.  Weights further down lose one per halving (in that
+// block alone); a tile with values below 2^-31 of their dim's scale (at 2^-31
+// they are off by 2^-20 at most), or with a scale that shrinks by more than
+// that, goes to ap_rows_f32 too, and so does one whose sums are not finite
+// (infinities and NaN turn into NaN here).
 //
 // Data movement: a block's K and V rows are loaded into registers one block
 // ahead of the conversion, converted by all four waves and stored as f16 in
@@ -379,14 +380,15 @@ __device__ __forceinline__ void ap_split(float x0, float x1, float minus_one, ui
     lo = __builtin_bit_cast(uint32_t, r);
 }
 
-// x0, x1, given times 2^11 -> packed f16 (hi) and 2^11 times what hi leaves
-// (lo): lo's smallest step is then 2^-35 of x's unit instead of 2^-24.  Two
+// x0, x1, given times 2^12 -> packed f16 (hi) and 2^12 times what hi leaves
+// (lo; at most 2^15 for |x| up to 2^15): lo's smallest step is then 2^-36 of
+// x's unit instead of 2^-24.  Two
 // v_fma_mix{lo,hi}_f16 per value.
 struct ApExt {
-    float down, neg;   // 2^-11 and -2^11 in registers that the compiler knows nothing of
+    float down, neg;   // 2^-12 and -2^12 in registers that the compiler knows nothing of
 };
 __device__ __forceinline__ ApExt ap_ext() {
-    ApExt e{0x1p-11f, -0x1p11f};
+    ApExt e{0x1p-12f, -0x1p12f};
     asm("" : "+s"(e.down), "+s"(e.neg));
     return e;
 }
@@ -414,7 +416,7 @@ __device__ __forceinline__ float ap_unscale(uint32_t e) { return __builtin_bit_c
 constexpr int AP_KQ = 14, AP_V = 14;
 constexpr int AP_P = 2;               // the largest p before its scale: its exponents are then near 0, where f32 is finest
 constexpr uint32_t AP_SCORE = 18;     // log2 of the |k||q| from which scores are left to the f32 kernel
-constexpr uint32_t AP_SPREAD = 34;    // octaves below a dim's largest |v| that the split takes
+constexpr uint32_t AP_SPREAD = 31;    // octaves below a dim's largest |v| that the split takes
 
 template <int HD>
 struct ApRegs {
@@ -497,7 +499,7 @@ __device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, in
     }
     // The smallest of the thread's values that are not zero (2 |bits| - 1 orders
     // them with zero last).  Dims below 2^-87 are left to the f32 kernel too.
-    // Standard normal values come that far apart once in 10^10.
+    // Standard normal values come that far apart once in 10^9.
     uint32_t um = 0xFFFFFFFFu;
     #pragma unroll
     for (int j = 0; j < L::PP; j++) {
@@ -510,7 +512,7 @@ __device__ __forceinline__ void ap_convert(uint8_t* lds, const ApRegs<HD>& r, in
         reinterpret_cast<float*>(lds + L::VR)[HD * (n & 1) + d] = ratio;
         reinterpret_cast<float*>(lds + L::VS)[d] = ap_unscale<AP_V>(vu);
     }
-    const float vs = ap_scale<AP_V + 11>(vu);
+    const float vs = ap_scale<AP_V + 12>(vu);
     const ApExt ex = ap_ext();
     uint32_t hi[L::PP / 2], lo[L::PP / 2];
     #pragma unroll
@@ -618,7 +620,7 @@ __device__ __forceinline__ void ap_compute(const uint8_t* lds, int n, int j0, co
     for (int r = 0; r < 8; r++) {
         const float p0 = fast_exp2(__builtin_fmaf(sc[2 * r], qf, -pref)), p1 = fast_exp2(__builtin_fmaf(sc[2 * r + 1], qf, -pref));
         rs[r] = p0 + p1;
-        ap_split_ext(p0 * (float)(1 << (26 - AP_P)), p1 * (float)(1 << (26 - AP_P)), ex, ph[r], pl[r]);
+        ap_split_ext(p0 * (float)(1 << (27 - AP_P)), p1 * (float)(1 << (27 - AP_P)), ex, ph[r], pl[r]);
     }
     // (as a tree: a chain of sixteen rounds more)
     const float rsum = ((rs[0] + rs[1]) + (rs[2] + rs[3])) + ((rs[4] + rs[5]) + (rs[6] + rs[7]));
@@ -649,7 +651,7 @@ __device__ __forceinline__ void ap_compute(const uint8_t* lds, int n, int j0, co
             }
         #pragma unroll
         for (int u = 0; u < U; u++) {
-            d[u] *= 0x1p-11f;
+            d[u] *= 0x1p-12f;
             #pragma unroll
             for (int s = 0; s < 2; s++) d[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[u][s], bh[s], d[u], 0, 0, 0);
         }

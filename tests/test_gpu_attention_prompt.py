@@ -228,6 +228,22 @@ def test_values_beside_a_large_one(prompt_be, hd, big, where):
 
 
 @pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("octaves", [20, 26, 29, 31, 32, 33.5, 35])
+def test_values_of_one_size_beside_a_large_one(prompt_be, hd, octaves):
+    """All |V| between 1 and 2 but for one masked position, 2^octaves: up to 31
+    octaves the split holds them (to 2^-20 at worst), above that the f32
+    products take the tile.  Bar 2^-20 of the largest |V| for a value and as
+    much for the weights' own roundings (scores below 10 nats to 2^-22)."""
+    n_head, n_kv, q_len, at = 8, 2, 64, 50
+    r = np.random.default_rng(hd)
+    q, k = (r.standard_normal(s).astype(F32) for s in ((n_head, q_len, hd), (n_kv, q_len, hd)))
+    v = ((1 + r.random((n_kv, q_len, hd))) * r.choice([-1.0, 1.0], (n_kv, 1, hd))).astype(F32)
+    v[:, at] = F32(2.0 ** octaves)
+    out, ref = attend_f32(prompt_be, q, k, v, n_head), exact(q, k, v, n_head)
+    assert np.max(np.abs(out[:at] - ref[:at])) <= 2 * 2.0 * 2.0 ** -20
+
+
+@pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("case", ["1e6", "1e8", "1e30", "huge keys", "huge queries"])
 def test_keys_and_queries_beside_large_elements(prompt_be, hd, case):
     """A large key element that the queries do not touch (they are 0 there)
